@@ -158,6 +158,21 @@ def test_target_layer_mask_row_stride(cuda, cfg, M, prefix):
     assert norm_err(got["padded rows"], want) < 1e-2, norm_err(got["padded rows"], want)
 
 
+@pytest.mark.parametrize("M,prefix", [(3, 30), (20, 100), (64, 1000)])
+def test_target_layer_causal_equals_causal_mask(cuda, M, prefix):
+    """A block without a mask sees every cached key and its own earlier rows, in
+    every key chunk: the same bits as the causal mask given explicitly."""
+    layer = TargetLayer(SMALL, random_layer(SMALL, seed=M, device=cuda), cuda)
+    cache = KVCache(SMALL.num_kv_heads, SMALL.head_dim, prefix + M, torch.bfloat16, cuda)
+    g = torch.Generator(device=cuda).manual_seed(M)
+    cache.keys[0, :, :prefix] = torch.randn(cache.keys[0, :, :prefix].shape, generator=g, device=cuda).bfloat16()
+    cache.values[0, :, :prefix] = torch.randn(cache.values[0, :, :prefix].shape, generator=g, device=cuda).bfloat16()
+    x = torch.randn(M, SMALL.hidden_size, generator=g, device=cuda)
+    off = torch.tensor([prefix], dtype=torch.int32, device=cuda)
+    mask = torch.ones(M, prefix + M, dtype=torch.uint8).tril(prefix)
+    assert torch.equal(layer(x.clone(), cache, off), layer(x.clone(), cache, off, mask=mask))
+
+
 def test_target_layer_rejects_bad_shapes(cuda):
     dev = torch.device("cuda", 0)
     layer = TargetLayer(SMALL, random_layer(SMALL, device=dev), dev)

@@ -1116,7 +1116,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2,
   const bool rlive = vrow < QV;
   const int mrow = min(vrow, QVb - 1) / rep;
   const int lim = offset + mrow;
-  const int wlo = a.window > 0 ? offset + mrow - a.window : -0x7fffffff;
+  const int wlo = a.window > 0 ? offset + mrow - a.window : -1;  // keys <= wlo are hidden (no window: none)
   float m_r = -INFINITY, l_r = 0.f;
   af32x4 o[8];
 #pragma unroll
