@@ -357,7 +357,7 @@ int wc_kv_compact(void* const* k_layers, void* const* v_layers, int n_layers, in
 
 #define WC_MAX_DRAFTER_LAYERS 4
 #define WC_MAX_FEATURES 3
-#define WC_MAX_STEP_ROWS 16 /* rows per drafter launch; longer inputs are tiled by the host */
+#define WC_MAX_STEP_ROWS 16 /* rows of a pass with a device row count; longer inputs run as many-row passes */
 
 /* DrafterConfig fields the kernels need (python/woodcock/drafter.py:33-49;
  * include/woodcock/drafter.h:16-24). */
@@ -405,7 +405,9 @@ typedef struct wc_gumbel {
  * Host memory, [max_pos][D/2] each. */
 int wc_rope_table(float* cos_out, float* sin_out, int max_pos, int head_dim, float base);
 
-/* Device workspace for wc_drafter_fuse / wc_drafter_forward / wc_draft_head. */
+/* Device workspace for wc_drafter_fuse / wc_drafter_forward / wc_draft_head
+ * (passes over many rows keep split activations of up to 1024 rows in it:
+ * about 0.14 GB at the Qwen3-4B width). */
 size_t wc_drafter_workspace_bytes(const wc_drafter_dims* dims);
 
 /* g[r] = fc(concat_f RMS_f(tap_f[row r])) for r < rows (device count *n_rows_dev

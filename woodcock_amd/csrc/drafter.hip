@@ -20,6 +20,7 @@
 #include "gemv.h"
 #include "gemvf.h"
 #include "gemv1s.h"
+#include "wide.h"
 
 namespace wc {
 
@@ -38,10 +39,33 @@ struct DrafterWs {
   float* partial;
   float* gs_part;        // k-split few-row GEMV: partial tiles per (tile, piece)
   unsigned int* gs_ctr;  // and one counter line per tile
+  uint16_t* planes_in;   // many-row passes: split activations of the projections' inputs,
+  uint16_t* planes_act;  // of the MLP's (or the fuse's) wide input,
+  float* wide_qkv;       // and fp32 rows
+  float* wide_q;
+  float* wide_h1;
   size_t bytes;
 };
 
 static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+
+// Rows of one many-row pass (longer inputs run several): 1024 rows fill the GPU
+// with tiles of the narrowest projection while the workspace stays near 0.14 MB
+// per row (Qwen3-4B shape).
+constexpr int kWideRows = 1024;
+
+// Rows above which a pass without a device row count or a mask goes to the
+// many-row path.  Fuse + layer at context 600, few-row kernels against the
+// many-row path: Qwen3-1.7B shape 8 rows 105 / 144 us, 9 rows 180 / 144 us (nine
+// rows leave the VALU GEMV); Qwen3-4B shape 4 rows 159 / 204 us, 5 rows 212 / 205
+// us, 8 rows 305 / 208 us (rows wider than 2048 leave it at five).
+static int wide_min_rows(const wc_drafter_dims& d) { return d.hidden > 2048 ? 4 : 8; }
+
+// Shapes the many-row GEMMs take: whole k steps of 32 and whole 16-row weight tiles.
+static bool wide_dims(const wc_drafter_dims& d) {
+  return d.hidden % 32 == 0 && d.inter % 32 == 0 && d.target_hidden % 32 == 0 && d.heads * d.head_dim % 32 == 0 &&
+         d.kv_heads * d.head_dim % 16 == 0;
+}
 
 static DrafterWs drafter_ws(const wc_drafter_dims& d, void* base) {
   DrafterWs w{};
@@ -66,6 +90,15 @@ static DrafterWs drafter_ws(const wc_drafter_dims& d, void* base) {
                                             (d.head_dim + 2)));
   w.gs_part = reinterpret_cast<float*>(take(4 * static_cast<size_t>(kGsMaxPieces) * kGsPieceFloats));
   w.gs_ctr = reinterpret_cast<unsigned int*>(take(4 * kCounterStride * static_cast<size_t>(kGsMaxPieces)));
+  if (wide_dims(d)) {
+    const size_t WR = kWideRows, nq = static_cast<size_t>(d.heads) * d.head_dim, hid = d.hidden;
+    w.planes_in = reinterpret_cast<uint16_t*>(take(wide_plane_bytes(WR, std::max(2 * hid, nq))));
+    w.planes_act = reinterpret_cast<uint16_t*>(take(wide_plane_bytes(
+        WR, std::max(static_cast<size_t>(d.inter), static_cast<size_t>(d.num_features) * d.target_hidden))));
+    w.wide_qkv = reinterpret_cast<float*>(take(4 * WR * nqkv));
+    w.wide_q = reinterpret_cast<float*>(take(4 * WR * nq));
+    w.wide_h1 = reinterpret_cast<float*>(take(4 * WR * hid));
+  }
   w.bytes = off;
   return w;
 }
@@ -715,6 +748,48 @@ int fuse_gemv_args(const wc_drafter_dims* dims, const wc_drafter_weights* w, con
 }
 }  // namespace wc
 
+namespace wc {
+// The fuse of many rows: the taps normalised into planes of num_features
+// segments, one GEMM per pass of kWideRows rows.
+static int fuse_wide(const wc_drafter_dims& d, const wc_drafter_weights& w, const void* const* taps, int tap_dtype,
+                     int64_t tap_ld, const int32_t* tap_rows_dev, int tap_rows, int rows, float* g_out, int64_t g_ld,
+                     const DrafterWs& ws, hipStream_t s) {
+  const int nf = d.num_features, Dt = d.target_hidden;
+  for (int t0 = 0; t0 < rows; t0 += kWideRows) {
+    const int tr = std::min(kWideRows, rows - t0);
+    WidePrepArgs p{};
+    p.n_seg = nf;
+    p.M = tr;
+    p.eps = d.eps;
+    p.xa = ws.planes_act;
+    p.steps = nf * Dt / 32;
+    for (int f = 0; f < nf; ++f) {
+      WC_REQUIRE(taps[f] != nullptr && al16(taps[f]), "wc_drafter_fuse: tap %d is NULL or not 16-byte aligned", f);
+      p.seg[f].x = static_cast<const char*>(taps[f]) + (tap_rows_dev ? 0 : t0 * tap_ld * (tap_dtype ? 2 : 4));
+      p.seg[f].ld = tap_ld;
+      p.seg[f].bf16 = tap_dtype == WC_BF16;
+      p.seg[f].row_idx = tap_rows_dev ? tap_rows_dev + t0 : nullptr;
+      p.seg[f].max_row = tap_rows_dev ? tap_rows : 0;
+      p.seg[f].gain = u16(w.feature_norm[f]);
+      p.seg[f].K = Dt;
+    }
+    if (int rc = launch_wide_prep(p, s)) return rc;
+    WideArgs g{};
+    g.xa = ws.planes_act;
+    g.steps = g.steps0 = nf * Dt / 32;
+    g.w[0][0] = u16(w.fc);
+    g.ldw = static_cast<int64_t>(nf) * Dt;
+    g.n_seg = 1;
+    g.M = tr;
+    g.N = d.hidden;
+    g.y = g_out + t0 * g_ld;
+    g.ldy = g_ld;
+    if (int rc = launch_wide_gemm(g, kWideStore, s)) return rc;
+  }
+  return WC_OK;
+}
+}  // namespace wc
+
 extern "C" {
 
 int wc_drafter_fuse(const wc_drafter_dims* dims, const wc_drafter_weights* w, const void* const* taps, int tap_dtype,
@@ -734,6 +809,10 @@ int wc_drafter_fuse(const wc_drafter_dims* dims, const wc_drafter_weights* w, co
   auto s = reinterpret_cast<hipStream_t>(stream);
   const int nf = dims->num_features, Dt = dims->target_hidden;
   const DrafterWs ws = drafter_ws(*dims, workspace);  // NULL workspace: no k split
+  // up to WC_MAX_STEP_ROWS rows the sums stay those of a pass with a device row
+  // count (a chain round fuses the same rows either way)
+  if (rows > WC_MAX_STEP_ROWS && workspace && wide_dims(*dims) && al16(g_out))
+    return fuse_wide(*dims, *w, taps, tap_dtype, tap_ld, tap_rows_dev, tap_rows, rows, g_out, g_ld, ws, s);
   for (int t0 = 0; t0 < rows; t0 += WC_MAX_STEP_ROWS) {
     const int tr = std::min(WC_MAX_STEP_ROWS, rows - t0);
     GemvArgs g = gemv_defaults();
@@ -776,6 +855,215 @@ struct PendTok {
   int32_t* tok;
   int32_t* row;
 };
+
+// A forward over many rows: passes of kWideRows rows, each projection one GEMM
+// over planes.  head_dim 128: q / k norm, RoPE and the append in one launch,
+// then attention over the cache by 64 query vectors per block; other head
+// sizes take the decode attention over row tiles.  No row count on the device
+// and no mask (those passes are a few rows).
+static int forward_wide(const wc_drafter_dims& d, const wc_drafter_weights& w, const int32_t* tokens_dev,
+                        const float* feat, int64_t feat_ld, const int32_t* feat_row_dev, int feat_row_add, int rows,
+                        void* const* k_cache, void* const* v_cache, int kv_dtype, int capacity,
+                        const int32_t* offset_dev, int offset_add, const int32_t* positions_dev, float* hidden_out,
+                        float* out_out, int32_t* advance_dev, const DrafterWs& ws, int splits, int tile_rows,
+                        hipStream_t s) {
+  const int H = d.heads, Hk = d.kv_heads, D = d.head_dim, nq = H * D, nk = Hk * D, nqkv = nq + 2 * nk;
+  const bool flash = D == 128 && static_cast<int64_t>(Hk) * capacity < (int64_t{1} << 31);
+  for (int t0 = 0; t0 < rows; t0 += kWideRows) {
+    const int tr = std::min(kWideRows, rows - t0);
+    float* hid = hidden_out + static_cast<int64_t>(t0) * d.hidden;
+    for (int li = 0; li < d.num_layers; ++li) {
+      const wc_layer_weights& L = w.layers[li];
+      const bool gathered = li == 0 && feat_row_dev;
+      const float* x = li > 0 ? hid : feat + (gathered ? 0 : t0 * feat_ld);
+      const int64_t ldx = li > 0 ? d.hidden : feat_ld;
+      const int32_t* xrow = gathered ? feat_row_dev + t0 : nullptr;
+
+      // 1. QKV over the normed input and, with the token stream, the normed embedding rows
+      WidePrepArgs p{};
+      p.n_seg = L.aux_norm ? 2 : 1;
+      p.M = tr;
+      p.eps = d.eps;
+      p.xa = ws.planes_in;
+      p.steps = p.n_seg * d.hidden / 32;
+      p.seg[0].x = x;
+      p.seg[0].ld = ldx;
+      p.seg[0].row_idx = xrow;
+      p.seg[0].row_add = xrow ? feat_row_add : 0;
+      p.seg[0].gain = u16(L.in_norm);
+      p.seg[0].K = d.hidden;
+      p.seg[1].x = w.embed;
+      p.seg[1].ld = d.hidden;
+      p.seg[1].bf16 = 1;
+      p.seg[1].row_idx = tokens_dev + t0;
+      p.seg[1].max_row = d.vocab;
+      p.seg[1].gain = u16(L.aux_norm);
+      p.seg[1].K = d.hidden;
+      if (int rc = launch_wide_prep(p, s)) return rc;
+      WideArgs g{};
+      g.xa = ws.planes_in;
+      g.steps = p.steps;
+      g.steps0 = d.hidden / 32;
+      g.w[0][0] = u16(L.q);
+      g.w[1][0] = u16(L.k);
+      g.w[2][0] = u16(L.v);
+      g.w[0][1] = u16(L.aux_q);
+      g.w[1][1] = u16(L.aux_k);
+      g.w[2][1] = u16(L.aux_v);
+      g.ldw = d.hidden;
+      g.n_seg = 3;
+      g.seg_start[1] = nq;
+      g.seg_start[2] = nq + nk;
+      g.M = tr;
+      g.N = nqkv;
+      g.y = ws.wide_qkv;
+      g.ldy = nqkv;
+      if (int rc = launch_wide_gemm(g, kWideStore, s)) return rc;
+
+      // 2. attention, its output as planes
+      if (flash) {
+        WideQkvArgs q{};
+        q.qkv = ws.wide_qkv;
+        q.H = H;
+        q.Hk = Hk;
+        q.rows = tr;
+        q.q_gain = u16(L.q_norm);
+        q.k_gain = u16(L.k_norm);
+        q.eps = d.eps;
+        q.rope_cos = w.rope_cos;
+        q.rope_sin = w.rope_sin;
+        q.rope_max = w.rope_max_pos;
+        q.positions = positions_dev ? positions_dev + t0 : nullptr;
+        q.offset_dev = offset_dev;
+        q.offset_add = offset_add + t0;
+        q.q = ws.wide_q;
+        q.kc = k_cache[li];
+        q.vc = v_cache[li];
+        q.cap = capacity;
+        if (int rc = launch_wide_qkv(q, kv_dtype, s)) return rc;
+        WideAttnArgs at{};
+        at.q = ws.wide_q;
+        at.ld_q = nq;
+        at.H = H;
+        at.Hk = Hk;
+        at.rows = tr;
+        at.k = k_cache[li];
+        at.v = v_cache[li];
+        at.ld_head = static_cast<int64_t>(capacity) * D;
+        at.ld_key = D;
+        at.keys = capacity;
+        at.offset_dev = offset_dev;
+        at.offset_add = offset_add + t0;
+        at.window = d.window;
+        at.scale = 1.f / sqrtf(static_cast<float>(D));
+        at.partial = ws.partial;
+        at.partial_floats = static_cast<size_t>(Hk) * kMaxSplits * kMaxQV * (D + 2);
+        at.planes = ws.planes_in;
+        if (int rc = launch_wide_attn(at, kv_dtype, s)) return rc;
+      } else {
+        for (int r0 = 0; r0 < tr; r0 += tile_rows) {
+          AttnArgs at{};
+          at.qkv = ws.wide_qkv + static_cast<int64_t>(r0) * nqkv;
+          at.ld_qkv = nqkv;
+          at.H = H;
+          at.Hk = Hk;
+          at.rows = std::min(tile_rows, tr - r0);
+          at.q_gain = u16(L.q_norm);
+          at.k_gain = u16(L.k_norm);
+          at.eps = d.eps;
+          at.scale = 1.f / sqrtf(static_cast<float>(D));
+          at.rope_cos = w.rope_cos;
+          at.rope_sin = w.rope_sin;
+          at.rope_max = w.rope_max_pos;
+          at.positions = positions_dev ? positions_dev + t0 + r0 : nullptr;
+          at.kc = k_cache[li];
+          at.vc = v_cache[li];
+          at.cap = capacity;
+          at.offset_dev = offset_dev;
+          at.offset_add = offset_add + t0 + r0;
+          at.window = d.window;
+          at.partial = ws.partial;
+          at.qv_ld = kMaxQV;
+          at.ctr = ws.attn_ctr;
+          at.out = ws.wide_q + static_cast<int64_t>(r0) * nq;
+          at.ld_out = nq;
+          if (int rc = launch_attention(at, D, kv_dtype, splits, s)) return rc;
+        }
+        WidePrepArgs pa{};
+        pa.n_seg = 1;
+        pa.M = tr;
+        pa.xa = ws.planes_in;
+        pa.steps = nq / 32;
+        pa.seg[0].x = ws.wide_q;
+        pa.seg[0].ld = nq;
+        pa.seg[0].K = nq;
+        if (int rc = launch_wide_prep(pa, s)) return rc;
+      }
+
+      // 3. h1 = h + W_o . o
+      g = WideArgs{};
+      g.xa = ws.planes_in;
+      g.steps = g.steps0 = nq / 32;
+      g.w[0][0] = u16(L.o);
+      g.ldw = nq;
+      g.n_seg = 1;
+      g.M = tr;
+      g.N = d.hidden;
+      g.res = x;
+      g.ldres = ldx;
+      g.res_row = xrow;
+      g.res_add = xrow ? feat_row_add : 0;
+      g.y = ws.wide_h1;
+      g.ldy = d.hidden;
+      if (int rc = launch_wide_gemm(g, kWideResidual, s)) return rc;
+
+      // 4. act = silu(W_gate . RMS_post(h1)) * (W_up . RMS_post(h1)), as planes
+      p = WidePrepArgs{};
+      p.n_seg = 1;
+      p.M = tr;
+      p.eps = d.eps;
+      p.xa = ws.planes_in;
+      p.steps = d.hidden / 32;
+      p.seg[0].x = ws.wide_h1;
+      p.seg[0].ld = d.hidden;
+      p.seg[0].gain = u16(L.post_norm);
+      p.seg[0].K = d.hidden;
+      if (int rc = launch_wide_prep(p, s)) return rc;
+      g = WideArgs{};
+      g.xa = ws.planes_in;
+      g.steps = g.steps0 = d.hidden / 32;
+      g.w[0][0] = u16(L.gate);
+      g.w[1][0] = u16(L.up);
+      g.ldw = d.hidden;
+      g.n_seg = 2;
+      g.M = tr;
+      g.N = d.inter;
+      g.planes = ws.planes_act;
+      if (int rc = launch_wide_gemm(g, kWideSiluPair, s)) return rc;
+
+      // 5. h = h1 + W_down . act
+      g = WideArgs{};
+      g.xa = ws.planes_act;
+      g.steps = g.steps0 = d.inter / 32;
+      g.w[0][0] = u16(L.down);
+      g.ldw = d.inter;
+      g.n_seg = 1;
+      g.M = tr;
+      g.N = d.hidden;
+      g.res = ws.wide_h1;
+      g.ldres = d.hidden;
+      g.y = hid;
+      g.ldy = d.hidden;
+      if (int rc = launch_wide_gemm(g, kWideResidual, s)) return rc;
+    }
+    if (out_out)
+      if (int rc = launch_wide_norm(hid, out_out + static_cast<int64_t>(t0) * d.hidden, tr, d.hidden,
+                                    u16(w.final_norm), d.eps, s))
+        return rc;
+  }
+  if (advance_dev) return launch_wide_advance(advance_dev, offset_dev, offset_add + rows, s);
+  return WC_OK;
+}
 
 static int drafter_forward_impl(const wc_drafter_dims* dims, const wc_drafter_weights* w, const int32_t* tokens_dev,
                                 const float* feat, int64_t feat_ld, const int32_t* feat_row_dev, int feat_row_add,
@@ -830,6 +1118,10 @@ static int drafter_forward_impl(const wc_drafter_dims* dims, const wc_drafter_we
   auto s = reinterpret_cast<hipStream_t>(stream);
   const int nqkv = (H + 2 * Hk) * D;
   const int splits = std::max(1, std::min(kMaxSplits, (capacity + kAttnChunkMax - 1) / kAttnChunkMax));
+  if (rows > wide_min_rows(d) && !n_rows_dev && !pend && !mask_dev && wide_dims(d))
+    return forward_wide(d, *w, tokens_dev, feat, feat_ld, feat_row_dev, feat_row_add, rows, k_cache, v_cache, kv_dtype,
+                        capacity, offset_dev, offset_add, positions_dev, hidden_out, out_out, advance_dev, ws, splits,
+                        tile_rows, s);
 
   for (int t0 = 0; t0 < rows; t0 += tile_rows) {
     const int tr = std::min(tile_rows, rows - t0);
