@@ -447,3 +447,33 @@ def test_one_launch_give_up_is_sticky_until_reinit(workload):
     reset_workspace(ws)
     for r in range(8):
         assert torch.equal(call(r), ref[r]), r
+
+
+@pytest.mark.parametrize("n,rows", [(4096, 3), (4097, 2), (151936, 62), (300001, 2)])
+@pytest.mark.parametrize("top_k,top_p", [(50, 1.0), (256, 0.9), (257, 0.97), (0, 0.9), (0, 0.9999)])
+def test_warping_over_several_blocks_per_row(cuda, n, rows, top_k, top_p):
+    """Rows over one and more vocabulary chunks, k at the edge of the listed path:
+    normal logits, a heavy-tailed row, a row of equal entries (more ties than the
+    candidate lists hold) and one with -inf entries; the same twice (the row
+    counters are left clean)."""
+    from woodcock_amd.sampling import SamplingParams
+
+    rng = np.random.default_rng(n + top_k)
+    lg = rng.standard_normal((rows, n)).astype(np.float32) * 3
+    lg[0] = (-1.1 * np.log(rng.permutation(n) + 1.0)).astype(np.float32)
+    lg[1] = 0.25
+    lg[1, rng.integers(0, n, 30)] = 2.0
+    lg[-1, ::2] = -np.inf
+    x = torch.from_numpy(lg).to(cuda)
+    sp = SamplingParams(0.8, top_k, top_p)
+    got = probs_from_logits(x, sp)
+    assert torch.equal(got > 0, probs_from_logits(x, sp) > 0)
+    got = got.cpu().numpy()
+    pick = [0, 1, rows - 1]
+    want = S.probs_from_logits(lg[pick], 0.8, top_k, top_p)
+    for r, w in zip(pick, want):
+        # the two fp32 row sums differ by up to 2^-20 relative, which moves the
+        # cumulative mass by as much: that many entries of the boundary's size
+        assert np.count_nonzero((got[r] > 0) != (w > 0)) <= 1 + 2.0 ** -20 / w[w > 0].min(), r
+        both = (got[r] > 0) & (w > 0)
+        np.testing.assert_allclose(got[r][both], w[both], rtol=1e-5)

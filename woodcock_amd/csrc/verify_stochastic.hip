@@ -1243,7 +1243,8 @@ __global__ __launch_bounds__(kStThreads) void k_stoch_fused(StochArgs a, int nch
 // for k = 1..j, so only the normalisers (div_k, s_k) need vocabulary-wide sums.
 // q is zero outside the head rows, so each rejection's sums run over the head
 // rows and the entries outside them contribute (sum of their p) / prod div_k.
-// One block walks the tree (k_tree_walk); a grid over the vocabulary then sums
+// k_tree_sums forms every sum and lookup known beforehand, one block walks the
+// tree (k_tree_walk); a grid over the vocabulary then sums
 // the final distribution chunk by chunk and the last block locates the draw
 // (k_tree_sample).
 
@@ -1257,6 +1258,14 @@ struct TreeState {
   double s[WC_MAX_NODES];
 };
 static_assert(sizeof(TreeState) <= kTreeStateBytes, "tree state exceeds its workspace slot");
+
+// What the accept test of a node needs at its parent
+struct TreeNode {
+  int32_t row;  // head row of its token, -1: outside the draft vocabulary
+  float p, q;   // target / raw draft probability of the token
+  int32_t pad;
+};
+static_assert(sizeof(TreeNode) * WC_MAX_NODES + 4 * kTreeParts <= kTreeNodesBytes, "tree nodes exceed their slot");
 
 struct TreeArgs {
   const float* p;  // [rows][ld_p] target probabilities per node
@@ -1276,6 +1285,10 @@ struct TreeArgs {
   int purpose;
   TreeState* st;
   double* chunk_data;  // [kMaxVocabChunks]
+  double* sums;        // [WC_MAX_NODES][kTreeParts][3]
+  TreeNode* nodes;     // [WC_MAX_NODES]
+  int32_t* bad_parts;  // [kTreeParts]
+  int32_t* chunk_rows; // [kMaxVocabChunks + 1]
   unsigned int* counter;
   wc_verdict* verdict;
 };
@@ -1293,28 +1306,126 @@ __device__ __forceinline__ double tree_chain(double p, double q, int tok, int j,
   return p;
 }
 
-__device__ __forceinline__ double block_sum_tw(double v, double* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = v;
-  __syncthreads();
-  double t = 0.0;
-  for (int w = 0; w < kTwThreads / kWave; ++w) t += red[w];
-  return t;
+// Everything of the walk that does not depend on its decisions, over (part,
+// node) blocks: each node's lookups at its parent (part 0; a wave searches d2t
+// 64 ways at a time), the sums of the nodes with children, and on the root's
+// blocks the checks of d2t and its chunk table.  One block walking the tree
+// made the sums of every node it came to over the whole vocabulary and searched
+// d2t one step at a time: 166 us for a 60-node tree of 151,936 entries.
+__global__ __launch_bounds__(kStThreads) void k_tree_sums(TreeArgs a) {
+  __shared__ double red[kStThreads / kWave];
+  const int t = threadIdx.x, part = blockIdx.x, v = blockIdx.y, parts = gridDim.x;
+  const int N = a.count ? min(max(*a.count, 0), a.rows) : a.rows;
+  if (v == 0) {
+    StochArgs sa{};
+    sa.vocab = a.vocab;
+    sa.head_rows = a.head_rows;
+    sa.d2t = a.d2t;
+    sa.chunk_rows = a.chunk_rows;
+    const int per = (a.head_rows + parts - 1) / parts, rb = part * per, re = min(a.head_rows, rb + per);
+    int bad = 0;
+    if (a.head_rows > 0) {
+      chunk_table(sa, rb, re);
+      if (a.d2t) bad = d2t_bad(sa, rb, re);
+    }
+    bad = __syncthreads_or(bad);
+    if (t == 0) a.bad_parts[part] = bad;
+  }
+  if (v >= N || !a.q) return;
+  if (part == 0 && v > 0 && t < kWave) {
+    const int par = a.parents[v], x = a.tokens[v];
+    TreeNode nd{-1, 0.f, 0.f, 0};
+    if (par >= 0 && par < v && x >= 0 && x < a.vocab) {  // (an invalid tree is reported by the walk)
+      int r = x < a.head_rows ? x : -1;
+      if (a.d2t) {  // the first row with d2t >= x lies in [lo, lo + len]
+        int lo = 0, len = a.head_rows;
+        while (len > 0) {
+          const int step = (len + kWave - 1) / kWave, at = lo + t * step;
+          const int m = __popcll(__ballot(t * step < len && a.d2t[min(at, a.head_rows - 1)] < x));
+          // the entries at lo, lo + step, ..: m of them below x (d2t ascending)
+          if (m == 0) {
+            len = 0;
+          } else {
+            const int first = lo + (m - 1) * step + 1;
+            len = min(lo + len, lo + m * step) - first;
+            lo = first;
+          }
+        }
+        r = lo < a.head_rows && a.d2t[lo] == x ? lo : -1;
+      }
+      const int qrow = a.q_rows ? a.q_rows[par] : par;
+      nd.row = r;
+      nd.p = a.p[static_cast<int64_t>(par) * a.ld_p + x];
+      if (r >= 0 && (!a.q_rows || (qrow >= 0 && qrow < a.q_count))) nd.q = a.q[static_cast<int64_t>(qrow) * a.ld_q + r];
+    }
+    if (t == 0) a.nodes[v] = nd;
+  }
+  // the sums, for nodes with children
+  const bool kid = t < N && t < WC_MAX_NODES && a.parents[min(t, N - 1)] == v;
+  if (!__syncthreads_or(kid ? 1 : 0)) return;
+  const int qrow = a.q_rows ? a.q_rows[v] : v;
+  if (a.q_rows && (qrow < 0 || qrow >= a.q_count)) return;
+  const float* pr = a.p + static_cast<int64_t>(v) * a.ld_p;
+  const float* qr = a.q + static_cast<int64_t>(qrow) * a.ld_q;
+  constexpr int kB = 8;
+  double sq = 0.0, sph = 0.0, spa = 0.0;
+  {
+    const int per = (a.head_rows + parts - 1) / parts, rb = part * per, re = min(a.head_rows, rb + per);
+    for (int r0 = rb + t; r0 < re; r0 += kStThreads * kB) {
+      float qv[kB], pv[kB];
+      int id[kB];
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const int r = min(r0 + u * kStThreads, a.head_rows - 1);
+        qv[u] = qr[r];
+        id[u] = a.d2t ? min(max(a.d2t[r], 0), a.vocab - 1) : r;
+      }
+#pragma unroll
+      for (int u = 0; u < kB; ++u) pv[u] = pr[id[u]];
+#pragma unroll
+      for (int u = 0; u < kB; ++u)
+        if (r0 + u * kStThreads < re) {
+          sq += static_cast<double>(qv[u]);
+          sph += static_cast<double>(pv[u]);
+        }
+    }
+  }
+  {
+    const int per = (a.vocab + parts - 1) / parts, rb = part * per, re = min(a.vocab, rb + per);
+    for (int i0 = rb + t; i0 < re; i0 += kStThreads * kB) {
+      float pv[kB];
+#pragma unroll
+      for (int u = 0; u < kB; ++u) pv[u] = pr[min(i0 + u * kStThreads, a.vocab - 1)];
+#pragma unroll
+      for (int u = 0; u < kB; ++u)
+        if (i0 + u * kStThreads < re) spa += static_cast<double>(pv[u]);
+    }
+  }
+  sq = block_sum_f64(sq, red);
+  sph = block_sum_f64(sph, red);
+  spa = block_sum_f64(spa, red);
+  if (t == 0) {
+    double* o = a.sums + (static_cast<int64_t>(v) * kTreeParts + part) * 3;
+    o[0] = sq;
+    o[1] = sph;
+    o[2] = spa;
+  }
 }
 
-__device__ __forceinline__ int head_row_of(const TreeArgs& a, int x) {
-  if (!a.d2t) return x < a.head_rows ? x : -1;
-  const int r = lower_bound_i32(a.d2t, a.head_rows, x);
-  return (r < a.head_rows && a.d2t[r] == x) ? r : -1;
-}
+// Head rows a thread of the walk holds (16 k over the block); wider draft
+// vocabularies map the rest from memory at every rejection.
+constexpr int kTwHold = 16;
 
 __global__ __launch_bounds__(kTwThreads) void k_tree_walk(TreeArgs a) {
-  __shared__ double red[kTwThreads / kWave];
+  __shared__ int s_id[kTwHold * kTwThreads];
+  __shared__ float s_q[kTwHold * kTwThreads];
+  __shared__ double red[3][kTwThreads / kWave];
   __shared__ int s_x[WC_MAX_NODES], s_mode[WC_MAX_NODES], s_path[WC_MAX_NODES];
+  __shared__ int s_par[WC_MAX_NODES], s_tok[WC_MAX_NODES];
+  __shared__ TreeNode s_node[WC_MAX_NODES];
+  __shared__ double s_sum[WC_MAX_NODES][3];
   __shared__ double s_div[WC_MAX_NODES], s_s[WC_MAX_NODES];
   __shared__ int s_bad, s_acc, s_nu;
-  __shared__ unsigned long long s_kids;
   const int t = threadIdx.x;
   const int N = a.count ? *a.count : a.rows;
   const bool n_ok = N >= 1 && N <= a.rows;
@@ -1326,55 +1437,67 @@ __global__ __launch_bounds__(kTwThreads) void k_tree_walk(TreeArgs a) {
   __syncthreads();
   if (n_ok) {  // parents[0] = -1, 0 <= parents[i] < i, tokens inside the vocabulary, d2t ascending
     int bad = 0;
-    for (int i = t; i < N; i += kTwThreads) {
-      const int par = a.parents[i], tok = a.tokens[i];
-      if (i == 0 ? par != -1 : (par < 0 || par >= i)) bad = 1;
+    if (t < N) {
+      const int par = a.parents[t], tok = a.tokens[t];
+      if (t == 0 ? par != -1 : (par < 0 || par >= t)) bad = 1;
       if (tok < 0 || tok >= a.vocab) bad = 1;
-      if (a.q_rows && (a.q_rows[i] < 0 || a.q_rows[i] >= a.q_count)) bad = 1;
+      if (a.q_rows && (a.q_rows[t] < 0 || a.q_rows[t] >= a.q_count)) bad = 1;
+      s_par[t] = par;
+      s_tok[t] = tok;
+      if (a.q) s_node[t] = a.nodes[t];
     }
-    if (a.d2t)
-      for (int r = t; r < a.head_rows; r += kTwThreads) {
-        const int x = a.d2t[r];
-        if (x < 0 || x >= a.vocab || (r + 1 < a.head_rows && a.d2t[r + 1] <= x)) bad = 1;
-      }
+    if (t < kTreeParts && a.bad_parts[t]) bad = 1;
+    if (a.q && t / 4 < N && t % 4 < 3) {  // a node's sum: its parts in order
+      double s = 0.0;
+#pragma unroll
+      for (int q = 0; q < kTreeParts; ++q) s += a.sums[(static_cast<int64_t>(t / 4) * kTreeParts + q) * 3 + t % 4];
+      s_sum[t / 4][t % 4] = s;
+    }
     if (bad) s_bad = 1;
   }
   __syncthreads();
   const bool bad = s_bad != 0;
+  // token ids of the held head rows, each read by the thread that wrote it
+#pragma unroll
+  for (int e = 0; e < kTwHold; ++e) {
+    const int r = max(min(t + e * kTwThreads, a.head_rows - 1), 0);
+    s_id[e * kTwThreads + t] = !bad && a.d2t && a.q ? a.d2t[r] : r;
+  }
   int v = 0, plen = 0, j = 0;
   double Q = 1.0;
   while (!bad) {
-    if (t < kWave) {
-      const unsigned long long m = __ballot(t < N && a.parents[min(t, N - 1)] == v);
-      if (t == 0) s_kids = m;
-    }
-    __syncthreads();
-    unsigned long long kids = s_kids;
+    unsigned long long kids = __ballot(t % kWave < N && s_par[min(t % kWave, N - 1)] == v);
     j = 0;
     if (kids == 0) break;  // a leaf: the draw is from p[v]
-    // node sums: Q, the target mass on the head rows and on the whole vocabulary
     const float* pr = a.p + static_cast<int64_t>(v) * a.ld_p;
     const float* qr = a.q + static_cast<int64_t>(a.q_rows ? a.q_rows[v] : v) * a.ld_q;
-    double sq = 0.0, sph = 0.0, spa = 0.0;
-    for (int r = t; r < a.head_rows; r += kTwThreads) {
-      sq += static_cast<double>(qr[r]);
-      sph += static_cast<double>(pr[a.d2t ? a.d2t[r] : r]);
+    Q = s_sum[v][0];
+    const double p_out = s_sum[v][2] - s_sum[v][1];  // target mass where q = 0
+    // the held head rows: p after the rejections so far and the raw q, which
+    // after j rejections is q / D, D the raw mass of the rows not rejected (the
+    // renormalisations telescope); requested before the first test
+    float pv[kTwHold];
+    {
+      float qv[kTwHold];
+#pragma unroll
+      for (int e = 0; e < kTwHold; ++e) {
+        qv[e] = qr[min(t + e * kTwThreads, a.head_rows - 1)];
+        pv[e] = pr[s_id[e * kTwThreads + t]];
+      }
+#pragma unroll
+      for (int e = 0; e < kTwHold; ++e) s_q[e * kTwThreads + t] = qv[e];
     }
-    for (int i = t; i < a.vocab; i += kTwThreads) spa += static_cast<double>(pr[i]);
-    Q = block_sum_tw(sq, red);
-    const double p_head = block_sum_tw(sph, red);
-    const double p_out = block_sum_tw(spa, red) - p_head;  // mass where q = 0
-    double divprod = 1.0;
+    double hp[kTwHold];
+    double divprod = 1.0, D = Q;
     int accepted = -1;
     while (kids != 0) {
       const int c = __builtin_ctzll(kids);
       kids &= kids - 1;
-      const int x = a.tokens[c];
+      const int x = s_tok[c], rx = s_node[c].row;
       if (t == 0) {  // the accept test at x after j rejections
-        const int rx = head_row_of(a, x);
-        const double q0 = (rx >= 0 && Q > 0.0) ? static_cast<double>(qr[rx]) / Q : 0.0;
+        const double q0 = (rx >= 0 && Q > 0.0) ? static_cast<double>(s_node[c].q) / Q : 0.0;
         double qx;
-        const double px = tree_chain(static_cast<double>(pr[x]), q0, x, j, s_x, s_mode, s_div, s_s, qx);
+        const double px = tree_chain(static_cast<double>(s_node[c].p), q0, x, j, s_x, s_mode, s_div, s_s, qx);
         int acc = -1;
         if (qx > 0.0) {
           const double u = philox_uniform(a.seed, round, a.purpose, static_cast<unsigned long long>(s_nu++));
@@ -1385,20 +1508,49 @@ __global__ __launch_bounds__(kTwThreads) void k_tree_walk(TreeArgs a) {
       __syncthreads();
       accepted = s_acc;
       if (accepted >= 0) break;
-      // rejection j + 1: residual mass, current p mass and the renormalising q mass
+      // rejection j + 1: residual mass, current p mass and the raw q mass left
+      if (j == 0)
+#pragma unroll
+        for (int e = 0; e < kTwHold; ++e)
+          hp[e] = t + e * kTwThreads < a.head_rows ? static_cast<double>(pv[e]) : 0.0;
       double z = 0.0, ps = 0.0, ss = 0.0;
-      for (int r = t; r < a.head_rows; r += kTwThreads) {
+#pragma unroll
+      for (int e = 0; e < kTwHold; ++e) {
+        const int r = t + e * kTwThreads;
+        const float qv = s_q[e * kTwThreads + t];
+        if (r < a.head_rows && r != rx) ss += static_cast<double>(qv);
+        // a row that has no target mass left has none after this (a wave of them
+        // skips the divisions: most rows, after top-k or top-p)
+        if (__ballot(hp[e] > 0.0) != 0) {
+          ps += hp[e];
+          z += fmax(hp[e] - (D > 0.0 ? static_cast<double>(qv) / D : 0.0), 0.0);
+        }
+      }
+      for (int r = t + kTwHold * kTwThreads; r < a.head_rows; r += kTwThreads) {
         const int tok = a.d2t ? a.d2t[r] : r;
         const double q0 = Q > 0.0 ? static_cast<double>(qr[r]) / Q : 0.0;
         double qj;
         const double pj = tree_chain(static_cast<double>(pr[tok]), q0, tok, j, s_x, s_mode, s_div, s_s, qj);
         z += fmax(pj - qj, 0.0);
         ps += pj;
-        ss += tok == x ? 0.0 : qj;
+        ss += tok == x || qj == 0.0 ? 0.0 : static_cast<double>(qr[r]);
       }
-      z = block_sum_tw(z, red);
-      ps = block_sum_tw(ps, red);
-      ss = block_sum_tw(ss, red);
+      z = wave_sum_dpp(z);
+      ps = wave_sum_dpp(ps);
+      ss = wave_sum_dpp(ss);
+      if (t % kWave == 0) {
+        red[0][t / kWave] = z;
+        red[1][t / kWave] = ps;
+        red[2][t / kWave] = ss;
+      }
+      __syncthreads();
+      z = ps = ss = 0.0;
+#pragma unroll
+      for (int w = 0; w < kTwThreads / kWave; ++w) {
+        z += red[0][w];
+        ps += red[1][w];
+        ss += red[2][w];
+      }
       const double outside = p_out / divprod;
       const double zt = outside + z;
       const bool normal = zt > 1e-12;
@@ -1407,11 +1559,22 @@ __global__ __launch_bounds__(kTwThreads) void k_tree_walk(TreeArgs a) {
         s_x[j] = x;
         s_mode[j] = normal ? 1 : 0;
         s_div[j] = div;
-        s_s[j] = ss;
+        s_s[j] = D > 0.0 ? ss / D : 0.0;
       }
-      __syncthreads();
       divprod *= div;
       ++j;
+      if (kids != 0 && ss > 0.0) {  // the map of this rejection
+#pragma unroll
+        for (int e = 0; e < kTwHold; ++e) {
+          if (__ballot(hp[e] > 0.0) != 0) {
+            const double d = normal ? hp[e] - (D > 0.0 ? static_cast<double>(s_q[e * kTwThreads + t]) / D : 0.0) : hp[e];
+            hp[e] = d > 0.0 ? d / div : 0.0;
+          }
+          if (t + e * kTwThreads == rx) s_q[e * kTwThreads + t] = 0.f;
+        }
+        D = ss;
+      }
+      __syncthreads();
       if (ss <= 0.0) break;
     }
     if (accepted < 0) break;  // every child rejected: the draw is from the current p at v
@@ -1466,12 +1629,11 @@ __global__ __launch_bounds__(kStThreads) void k_tree_sample(TreeArgs a) {
     __syncthreads();
     if (j > 0 && qr && Q > 0.0) {
       if (a.d2t) {
-        const int r0 = lower_bound_i32(a.d2t, a.head_rows, x0);
-        const int r1 = lower_bound_i32(a.d2t, a.head_rows, x0 + kVocabChunk);
-        for (int r = r0 + t; r < r1; r += kStThreads) qchunk[a.d2t[r] - x0] = static_cast<double>(qr[r]) / Q;
+        const int r0 = a.chunk_rows[c], r1 = a.chunk_rows[c + 1];
+        for (int r = r0 + t; r < r1; r += kStThreads) qchunk[qslot(a.d2t[r] - x0)] = static_cast<double>(qr[r]) / Q;
       } else {
         for (int k = t; k < kVocabChunk && x0 + k < a.head_rows; k += kStThreads)
-          qchunk[k] = static_cast<double>(qr[x0 + k]) / Q;
+          qchunk[qslot(k)] = static_cast<double>(qr[x0 + k]) / Q;
       }
     }
     __syncthreads();
@@ -1484,8 +1646,10 @@ __global__ __launch_bounds__(kStThreads) void k_tree_sample(TreeArgs a) {
     for (int e = 0; e < kPerThread; ++e) {
       const int k = t * kPerThread + e, x = x0 + k;
       double qo;
-      val[e] = x < a.vocab ? tree_chain(static_cast<double>(pxf[e]), qchunk[k], x, j, s_x, s_mode, s_div, s_s, qo)
-                           : 0.0;
+      // an entry without target mass keeps none through the map
+      val[e] = x < a.vocab && pxf[e] != 0.f
+                   ? tree_chain(static_cast<double>(pxf[e]), qchunk[qslot(k)], x, j, s_x, s_mode, s_div, s_s, qo)
+                   : 0.0;
     }
   };
   const int c = blockIdx.x, nchunks = gridDim.x;
@@ -1593,8 +1757,8 @@ __device__ __forceinline__ float warped(const ProbsArgs& a, uint32_t kth, float 
 
 // ------------------------------------------------------------------ top-k / top-p warping
 //
-// Radix select over 32-bit order keys in three digit passes (11, 11, 10 bits),
-// one block per row: each pass histograms the digit of the keys that match the
+// Radix select over 32-bit order keys in three digit passes (11, 11, 10 bits)
+// by one block: each pass histograms the digit of the keys that match the
 // digits fixed so far, weighted by 1 (top-k) or by the value (top-p, fp64
 // sums), and fixes the digit of the bin where the weight of all larger keys
 // first reaches the target.  Finds the k-th largest key exactly; for top-p the
@@ -1605,12 +1769,11 @@ constexpr int kRsPerThread = kRsBins / kStThreads;  // bins per thread
 
 // One pass: digit of the crossing bin; `need` (weight still to cover) and
 // `above` (weight of larger keys) are updated.  TOPP: key = bits(p), weight p;
-// else key = float_order(logit / T) (the division the softmax kernels use),
-// weight 1.  When fp64 rounding leaves the crossing just past the last
+// else key = float_order(value), weight 1.  val(i), i < n: the values.  When fp64 rounding leaves the crossing just past the last
 // nonempty bin (top-p only), that bin is taken: every remaining entry stays.
 // s_w: kStThreads / kWave + 2 doubles.
-template <bool TOPP>
-__device__ uint32_t rs_pass(const float* row, int n, float temp, int shift, int bits, uint32_t prefix,
+template <bool TOPP, class F>
+__device__ uint32_t rs_pass(const F& val, int n, int shift, int bits, uint32_t prefix,
                             uint32_t pmask, double& need, double& above, double* s_mass, unsigned* s_cnt,
                             double* s_w, uint32_t* s_digit) {
   const int t = threadIdx.x;
@@ -1621,8 +1784,8 @@ __device__ uint32_t rs_pass(const float* row, int n, float temp, int shift, int 
   }
   __syncthreads();
   for (int i = t; i < n; i += kStThreads) {
-    const float v = row[i];
-    const uint32_t key = TOPP ? __float_as_uint(v) : float_order(v / temp);
+    const float v = val(i);
+    const uint32_t key = TOPP ? __float_as_uint(v) : float_order(v);
     if ((key & pmask) == prefix) {
       const uint32_t d = (key >> shift) & (nb - 1);
       if (TOPP) atomicAdd(&s_mass[d], static_cast<double>(v));
@@ -1679,25 +1842,396 @@ __device__ uint32_t rs_pass(const float* row, int n, float temp, int shift, int 
   return d;
 }
 
-// top-k: the order key of the k-th largest logit / T of row blockIdx.x
-__global__ __launch_bounds__(kStThreads) void k_topk_key(ProbsArgs a, int k, uint32_t* keys) {
-  __shared__ double s_mass[kRsBins];
-  __shared__ unsigned s_cnt[kRsBins];
-  __shared__ double s_w[kStThreads / kWave + 2];
-  __shared__ uint32_t s_digit[2];
-  const int r = blockIdx.x;
-  const float* row = a.logits + static_cast<int64_t>(r) * a.ld;
-  double need = k, above = 0.0;
+// LDS of the radix select and of the block sums around it
+struct RsShared {
+  double mass[kRsBins];
+  unsigned cnt[kRsBins];
+  double w[kStThreads / kWave + 2];
+  uint32_t digit[2];
+};
+
+// The key where the weight of the larger keys first reaches `need`; `above`:
+// the weight of the keys above it.
+template <bool TOPP, class F>
+__device__ uint32_t rs_select(const F& val, int n, double need, double& above, RsShared& sh) {
   uint32_t prefix = 0, pmask = 0;
   const int shifts[3] = {21, 10, 0}, widths[3] = {11, 11, 10};
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    const uint32_t d = rs_pass<false>(row, a.n, a.temperature, shifts[q], widths[q], prefix, pmask, need, above,
-                                      s_mass, s_cnt, s_w, s_digit);
+    const uint32_t d =
+        rs_pass<TOPP>(val, n, shifts[q], widths[q], prefix, pmask, need, above, sh.mass, sh.cnt, sh.w, sh.digit);
     prefix |= d << shifts[q];
     pmask |= ((1u << widths[q]) - 1u) << shifts[q];
   }
-  if (threadIdx.x == 0) keys[r] = prefix;
+  return prefix;
+}
+
+// top-k: the order key of the k-th largest logit / T of row blockIdx.x (the
+// division the softmax kernels use); the path for k too large for k_topk_bound
+__global__ __launch_bounds__(kStThreads) void k_topk_key(ProbsArgs a, int k, uint32_t* keys) {
+  __shared__ RsShared sh;
+  const int r = blockIdx.x;
+  const float* row = a.logits + static_cast<int64_t>(r) * a.ld;
+  double above = 0.0;
+  const uint32_t key = rs_select<false>([&](int i) { return scaled(a, row[i]); }, a.n, k, above, sh);
+  if (threadIdx.x == 0) keys[r] = key;
+}
+
+// Which entries of a row the warp keeps: those with probability bits above
+// `key`, and of the ones equal to it those at index <= last; p is divided by `mass`.
+struct WarpSel {
+  uint32_t key;
+  int32_t last;
+  double mass;
+};
+static_assert(sizeof(WarpSel) * WC_MAX_NODES <= kWarpSelBytes, "warp results exceed their workspace slot");
+
+// The top-p boundary of n entries val(i) at row index idx(i) (any order),
+// `above` the mass of the row's entries that are larger than all of them: the
+// entries kept are those of the descending order (ties: lower index first)
+// whose exclusive cumulative mass is below top_p -- every entry above the
+// boundary value t, and of the entries equal to t the first
+// ceil((top_p - G) / t), G the mass above t.  The same result in every thread.
+template <class F, class I>
+__device__ WarpSel topp_select(const F& val, const I& idx, int n, double top_p, double above, RsShared& sh) {
+  const int t = threadIdx.x;
+  double G = above;
+  const uint32_t tk = rs_select<true>(val, n, top_p - above, G, sh);
+  const double tv = static_cast<double>(__uint_as_float(tk));
+  double eq = 0.0, mass = 0.0;
+  for (int i = t; i < n; i += kStThreads) {
+    const float v = val(i);
+    const uint32_t k = __float_as_uint(v);
+    if (k == tk) eq += 1.0;
+    if (k > tk) mass += static_cast<double>(v);
+  }
+  eq = block_sum_f64(eq, sh.w);
+  mass = block_sum_f64(mass, sh.w) + above;
+  const double keep_eq = tv > 0.0 ? fmax(1.0, ceil((top_p - G) / tv)) : 1.0;
+  WarpSel sel{tk, 0x7fffffff, 0.0};
+  if (keep_eq < eq) {  // the keep_eq-th smallest index among the equal entries, bit by bit
+    int lim = 0;
+    for (int b = 30; b >= 0; --b) {
+      const int cand = lim | 1 << b;
+      double c = 0.0;
+      for (int i = t; i < n; i += kStThreads)
+        if (__float_as_uint(val(i)) == tk && idx(i) < cand) c += 1.0;
+      if (block_sum_f64(c, sh.w) < keep_eq) lim = cand;
+    }
+    sel.last = lim;
+    sel.mass = mass + keep_eq * tv;
+  } else {
+    sel.mass = mass + eq * tv;
+  }
+  return sel;
+}
+
+// One of `total` blocks counting on a row's counter; true in the last, which resets it.
+__device__ __forceinline__ bool warp_last(unsigned int* ctr, unsigned int total) {
+  __shared__ bool s_last;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const bool last = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1;
+    if (last) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = last;
+  }
+  __syncthreads();
+  return s_last;
+}
+
+// Appends `item` of the threads with `on` to a row's list (positions past
+// kWarpList are counted, not stored).
+__device__ __forceinline__ void warp_append(bool on, unsigned long long item, unsigned int* count,
+                                            unsigned long long* list) {
+  const unsigned long long m = __ballot(on);
+  if (m == 0) return;
+  const int lane = threadIdx.x % kWave;
+  unsigned int base = 0;
+  if (lane == __builtin_ctzll(m))
+    base = __hip_atomic_fetch_add(count, static_cast<unsigned int>(__popcll(m)), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+  base = __builtin_amdgcn_readlane(base, __builtin_ctzll(m));
+  const unsigned int pos = base + __popcll(m & ((1ull << lane) - 1));
+  if (on && pos < kWarpList) atomic_store_u64(list + pos, item);
+}
+
+// top-k of up to kTopkMax entries by several blocks per row.  Any k entries give
+// a lower bound of the k-th largest, and the k-th largest of the maxima of many
+// groups is a close one (60 rows of 151,936, k 50: 51 candidates).  Launch 1
+// (several blocks per row): their group maxima; the row's last block
+// finds the k-th largest of them.  Launch 2: every entry below the bound is
+// written as 0, the others are listed, and the row's last block finishes the
+// list.  One block per row made three histogram passes over it: 569 us for 60
+// rows, and the softmax and top-p passes over rows of which k entries are left.
+constexpr int kTopkMax = 256;
+constexpr int kTopkList = 1024;  // candidates finished in LDS; more (ties) go through the radix select
+
+struct WarpArgs {
+  ProbsArgs a;
+  int k;              // 0: off
+  double top_p;       // 1: off
+  int span;           // entries of a row per block (a multiple of 4)
+  int groups;         // group maxima per block: a power of two
+  unsigned int *ctr, *count;  // [rows][kCounterStride]
+  uint32_t *maxima, *bound;   // [rows][kWarpGroups] of scaled logits; [rows]: the raw logits' lower bound
+  unsigned long long* list;   // [rows][kWarpList]
+  double* hist;               // [rows][parts][kWarpBins]
+  WarpSel* sel;
+  int parts;
+};
+
+// 16 entries of a thread from x0 on: four 16-byte loads where rows keep them
+// whole (VEC), else 16 strided ones; entry e is at x0 + warp_at<VEC>(e).
+template <bool VEC>
+__device__ __forceinline__ int warp_at(int e) {
+  return VEC ? (e / 4 * kStThreads + static_cast<int>(threadIdx.x)) * 4 + e % 4
+             : e * kStThreads + static_cast<int>(threadIdx.x);
+}
+template <bool VEC>
+__device__ __forceinline__ void warp_load(const float* lr, int x0, int n, float (&raw)[kPerThread]) {
+  if constexpr (VEC) {
+    float4 v[kPerThread / 4];
+#pragma unroll
+    for (int e = 0; e < kPerThread / 4; ++e)
+      v[e] = *reinterpret_cast<const float4*>(lr + min(x0 + warp_at<true>(4 * e), n - 4));
+#pragma unroll
+    for (int e = 0; e < kPerThread / 4; ++e) {
+      raw[4 * e] = v[e].x;
+      raw[4 * e + 1] = v[e].y;
+      raw[4 * e + 2] = v[e].z;
+      raw[4 * e + 3] = v[e].w;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e) raw[e] = lr[min(x0 + warp_at<false>(e), n - 1)];
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e) pin(raw[e]);
+  }
+}
+
+// float of an order key
+__device__ __forceinline__ float order_float(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(kStThreads) void k_topk_bound(WarpArgs w) {
+  const ProbsArgs& a = w.a;
+  const int t = threadIdx.x, r = blockIdx.y, b0 = blockIdx.x * w.span, b1 = min(a.n, b0 + w.span);
+  const float* lr = a.logits + static_cast<int64_t>(r) * a.ld;
+  uint32_t m = 0;  // (the scaling keeps the order: the maximum is taken over the raw logits)
+  for (int x0 = b0; x0 < b1; x0 += kVocabChunk) {
+    float raw[kPerThread];
+    warp_load<VEC>(lr, x0, a.n, raw);
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e)
+      if (x0 + warp_at<VEC>(e) < b1) m = max(m, float_order(raw[e]));
+  }
+  if (m != 0) m = float_order(scaled(a, order_float(m)));
+  const int lanes = kStThreads / w.groups;  // 1 .. 64
+  for (int o = 1; o < lanes; o <<= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), o)));
+  uint32_t* row = w.maxima + static_cast<int64_t>(r) * kWarpGroups;
+  if (t % lanes == 0) atomic_store_u32(row + blockIdx.x * w.groups + t / lanes, m);
+  if (!warp_last(w.ctr + r * kCounterStride, gridDim.x)) return;
+  // the k-th largest of the row's maxima, bit by bit
+  const int n = gridDim.x * w.groups;
+  uint32_t v[kWarpGroups / kStThreads];
+#pragma unroll
+  for (int e = 0; e < kWarpGroups / kStThreads; ++e) {
+    const int i = e * kStThreads + t;
+    v[e] = __hip_atomic_load(row + min(i, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (i >= n) v[e] = 0;
+  }
+  __shared__ int s_c[2][kStThreads / kWave];
+  uint32_t key = 0;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t cand = key | 1u << b;
+    int c = 0;
+#pragma unroll
+    for (int e = 0; e < kWarpGroups / kStThreads; ++e) c += __popcll(__ballot(v[e] >= cand));
+    if (t % kWave == 0) s_c[b & 1][t / kWave] = c;
+    __syncthreads();
+    int tot = 0;
+#pragma unroll
+    for (int q = 0; q < kStThreads / kWave; ++q) tot += s_c[b & 1][q];
+    if (tot >= w.k) key = cand;
+  }
+  // the smallest raw logit (as its order key) that scales to the bound or above:
+  // within a few steps of bound * T (wave 0, one step per lane), else bit by bit
+  if (t < kWave) {
+    const uint32_t guess = float_order(order_float(key) * a.temperature);
+    const uint32_t at = guess - kWave / 2 + t;
+    const unsigned long long ge = __ballot(float_order(scaled(a, order_float(at))) >= key);
+    const bool plain = key != 0 && guess > kWave && guess < 0xff000000u;
+    uint32_t lo = 0;
+    if (plain && ge != 0 && !(ge & 1)) {
+      lo = guess - kWave / 2 + __builtin_ctzll(ge);
+    } else {
+      for (int b = 31; b >= 0; --b) {
+        const uint32_t cand = lo | 1u << b;
+        if (float_order(scaled(a, order_float(cand - 1))) < key) lo = cand;
+      }
+    }
+    if (t == 0) w.bound[r] = lo;
+  }
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(kStThreads) void k_topk_finish(WarpArgs w) {
+  const ProbsArgs& a = w.a;
+  const int t = threadIdx.x, r = blockIdx.y, b0 = blockIdx.x * w.span, b1 = min(a.n, b0 + w.span);
+  const float* lr = a.logits + static_cast<int64_t>(r) * a.ld;
+  float* orow = a.out + static_cast<int64_t>(r) * a.ld_out;
+  const uint32_t bound = w.bound[r];
+  unsigned int* count = w.count + r * kCounterStride;
+  unsigned long long* list = w.list + static_cast<int64_t>(r) * kWarpList;
+  // an entry in the running: not below the bound, and not -inf (p = 0 either way)
+  auto candidate = [&](float v) { return float_order(v) >= bound && v != -INFINITY; };
+  for (int x0 = b0; x0 < b1; x0 += kVocabChunk) {
+    float raw[kPerThread];
+    warp_load<VEC>(lr, x0, a.n, raw);
+    // zeros for the others (the last block writes the candidates: no two blocks
+    // store to one entry)
+    bool on[kPerThread];
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e) on[e] = x0 + warp_at<VEC>(e) < b1 && candidate(raw[e]);
+#pragma unroll
+    for (int e = 0; e < kPerThread; e += 4) {
+      const int i = x0 + warp_at<VEC>(e);
+      if (VEC && i < b1 && !(on[e] || on[e + 1] || on[e + 2] || on[e + 3])) {
+        *reinterpret_cast<float4*>(orow + i) = float4{0.f, 0.f, 0.f, 0.f};
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int iu = x0 + warp_at<VEC>(e + u);
+          if (iu < b1 && !on[e + u]) orow[iu] = 0.f;
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e)
+      if (__ballot(on[e]) != 0) {
+        const float x = scaled(a, raw[e]);
+        warp_append(on[e], static_cast<unsigned long long>(__float_as_uint(x)) << 32 |
+                               static_cast<unsigned int>(x0 + warp_at<VEC>(e)), count, list);
+      }
+  }
+  if (!warp_last(w.ctr + r * kCounterStride, gridDim.x)) return;
+
+  __shared__ union {
+    RsShared rs;
+    struct {
+      float x[kTopkList];
+      int i[kTopkList];
+    } c;
+  } sh;
+  __shared__ double s_red[kStThreads / kWave];
+  __shared__ float s_max[kStThreads / kWave];
+  const int nc = static_cast<int>(__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  __syncthreads();
+  if (t == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  auto block_max = [&](float m) {
+    m = wave_max_dpp(m);
+    __syncthreads();
+    if (t % kWave == 0) s_max[t / kWave] = m;
+    __syncthreads();
+    float v = s_max[0];
+#pragma unroll
+    for (int q = 1; q < kStThreads / kWave; ++q) v = fmaxf(v, s_max[q]);
+    return v;
+  };
+  if (nc <= kTopkList) {
+    constexpr int PER = kTopkList / kStThreads;
+    float x[PER], p[PER];
+    int id[PER];
+    bool on[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int i = e * kStThreads + t;
+      const unsigned long long u = atomic_load_u64(list + min(i, kWarpList - 1));
+      on[e] = i < nc;
+      x[e] = on[e] ? __uint_as_float(static_cast<uint32_t>(u >> 32)) : -INFINITY;
+      id[e] = static_cast<int>(static_cast<uint32_t>(u));
+      sh.c.x[i] = x[e];
+    }
+    __syncthreads();
+    // ranks: an entry with at least k larger ones drops out (ties with the k-th stay)
+    float m = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      if (e * kStThreads >= nc) break;  // uniform
+      const uint32_t key = float_order(x[e]);
+      int larger = 0;
+      for (int j = 0; j < nc; ++j) larger += float_order(sh.c.x[j]) > key ? 1 : 0;
+      on[e] = on[e] && larger < w.k;
+      if (on[e]) m = fmaxf(m, x[e]);
+    }
+    const float M = block_max(m);
+    double s = 0.0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      p[e] = on[e] ? expf(x[e] - M) : 0.f;
+      s += static_cast<double>(p[e]);
+    }
+    const float S = static_cast<float>(block_sum_f64(s, s_red));
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      if (on[e]) p[e] = p[e] / S;
+    if (w.top_p < 1.0) {
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        sh.c.x[e * kStThreads + t] = on[e] ? p[e] : 0.f;
+        sh.c.i[e * kStThreads + t] = id[e];
+      }
+      __syncthreads();
+      // the mass before an entry in descending order, ties by index
+      double kept = 0.0;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        if (e * kStThreads >= nc) break;
+        double before = 0.0;
+        for (int j = 0; j < nc; ++j) {
+          const float q = sh.c.x[j];
+          const bool first = __float_as_uint(q) > __float_as_uint(p[e]) || (q == p[e] && sh.c.i[j] < id[e]);
+          before += first ? static_cast<double>(q) : 0.0;
+        }
+        on[e] = on[e] && before < w.top_p;
+        if (on[e]) kept += static_cast<double>(p[e]);
+      }
+      const double tot = block_sum_f64(kept, s_red);
+#pragma unroll
+      for (int e = 0; e < PER; ++e) p[e] = on[e] ? static_cast<float>(static_cast<double>(p[e]) / tot) : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      if (e * kStThreads + t < nc) orow[id[e]] = p[e];
+    return;
+  }
+  // many ties at the bound: the general selection over the whole row
+  double above = 0.0;
+  const uint32_t kth = rs_select<false>([&](int i) { return scaled(a, lr[i]); }, a.n, w.k, above, sh.rs);
+  float m = -INFINITY;
+  for (int i = t; i < a.n; i += kStThreads) m = fmaxf(m, warped(a, kth, lr[i]));
+  const float M = block_max(m);
+  auto e_of = [&](int i) {
+    const float v = warped(a, kth, lr[i]);
+    return v == -INFINITY ? 0.f : expf(v - M);
+  };
+  double s = 0.0;
+  for (int i = t; i < a.n; i += kStThreads) s += static_cast<double>(e_of(i));
+  const float S = static_cast<float>(block_sum_f64(s, s_red));
+  auto p_of = [&](int i) { return e_of(i) / S; };
+  WarpSel sel{0u, 0x7fffffff, 1.0};
+  if (w.top_p < 1.0) sel = topp_select(p_of, [](int i) { return i; }, a.n, w.top_p, 0.0, sh.rs);
+  for (int i = t; i < a.n; i += kStThreads) {
+    if (!candidate(lr[i])) continue;
+    const float v = p_of(i);
+    const uint32_t key = __float_as_uint(v);
+    const bool keep = key > sel.key || (key == sel.key && i <= sel.last);
+    orow[i] = w.top_p < 1.0 ? (keep ? static_cast<float>(static_cast<double>(v) / sel.mass) : 0.f) : v;
+  }
 }
 
 // (max, sum of exp(x - max)) of chunk blockIdx.x of row blockIdx.y
@@ -1826,65 +2360,190 @@ __global__ __launch_bounds__(kSrThreads) void k_softmax_row(ProbsArgs a) {
   }
 }
 
-// top-p on the written probabilities of row blockIdx.x, in place: keep the
-// entries of the descending order (ties: lower index first) whose exclusive
-// cumulative mass is below top_p -- every entry above the boundary value t, and
-// of the entries equal to t the first ceil((top_p - G) / t) -- then renormalise
-// by the kept mass (fp64).
-__global__ __launch_bounds__(kStThreads) void k_topp(ProbsArgs a, float top_p) {
-  __shared__ double s_mass[kRsBins];
-  __shared__ unsigned s_cnt[kRsBins];
-  __shared__ double s_w[kStThreads / kWave + 2];
-  __shared__ uint32_t s_digit[2];
-  const int r = blockIdx.x, t = threadIdx.x, n = a.n;
-  float* row = a.out + static_cast<int64_t>(r) * a.ld_out;
-  double need = top_p, above = 0.0;
-  uint32_t prefix = 0, pmask = 0;
-  const int shifts[3] = {21, 10, 0}, widths[3] = {11, 11, 10};
+// top-p over several blocks per row, in three launches after k_softmax_part (one
+// block per row made its radix passes with every zero added to one bin: 1.09 ms
+// for 60 rows of 151,936).  Probabilities are formed where they are read, so
+// they are written once: k_topp_hist sums each part's mass per bin;
+// k_topp_bound finds the bin where the mass reaches top_p
+// and lists its entries, which the row's last block selects from; k_topp_write
+// writes the row.
+
+// a row's softmax: M and S from the chunk partials, merged as k_softmax_write does
+struct RowSoftmax {
+  float M, S;
+  uint32_t kth;
+};
+__device__ __forceinline__ RowSoftmax row_softmax(const ProbsArgs& a, int r) {
+  __shared__ float s_M, s_S;
+  const int nch = (a.n + kVocabChunk - 1) / kVocabChunk;
+  const float* pp = a.part + static_cast<int64_t>(r) * kMaxVocabChunks * 2;
+  if (threadIdx.x < kWave) {
+    float m = -INFINITY;
+    for (int c = threadIdx.x; c < nch; c += kWave) m = fmaxf(m, pp[2 * c]);
+    m = wave_max_dpp(m);
+    float s = 0.f;
+    for (int c = threadIdx.x; c < nch; c += kWave) {
+      const float mc = pp[2 * c];
+      s += mc == -INFINITY ? 0.f : pp[2 * c + 1] * expf(mc - m);
+    }
+    s = wave_sum_dpp(s);
+    if (threadIdx.x == 0) {
+      s_M = m;
+      s_S = s;
+    }
+  }
+  __syncthreads();
+  return {s_M, s_S, kth_order(a, r)};
+}
+__device__ __forceinline__ float row_p(const ProbsArgs& a, const RowSoftmax& rs, float raw) {
+  const float v = warped(a, rs.kth, raw);
+  return v == -INFINITY ? 0.f : expf(v - rs.M) / rs.S;
+}
+
+// Bin of p's bits: 64 bins per octave below 1 (a heavy-tailed row puts ~1% of
+// its rank in one, which fits the list), everything under 2^-32 in bin 0.
+__device__ __forceinline__ uint32_t topp_bin(uint32_t key) {
+  return static_cast<uint32_t>(min(max(static_cast<int>(key >> 17) - ((127 - 32) << 6), 0), kWarpBins - 1));
+}
+constexpr int kToppBatch = 8;   // loads in flight per thread
+
+__global__ __launch_bounds__(kStThreads) void k_topp_hist(WarpArgs w) {
+  __shared__ double s_mass[kWarpBins];
+  const ProbsArgs& a = w.a;
+  const int t = threadIdx.x, r = blockIdx.y, per = (a.n + w.parts - 1) / w.parts;
+  const int b0 = blockIdx.x * per, b1 = min(a.n, b0 + per);
+  for (int b = t; b < kWarpBins; b += kStThreads) s_mass[b] = 0.0;
+  const RowSoftmax rs = row_softmax(a, r);  // (its barrier covers the bins)
+  const float* lr = a.logits + static_cast<int64_t>(r) * a.ld;
+  for (int i0 = b0 + t; i0 < b1; i0 += kStThreads * kToppBatch) {
+    float raw[kToppBatch];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const uint32_t d =
-        rs_pass<true>(row, n, 1.f, shifts[q], widths[q], prefix, pmask, need, above, s_mass, s_cnt, s_w, s_digit);
-    prefix |= d << shifts[q];
-    pmask |= ((1u << widths[q]) - 1u) << shifts[q];
-  }
-  const uint32_t tk = prefix;  // bits of the boundary value
-  const double tv = static_cast<double>(__uint_as_float(tk)), G = above;
-  // entries equal to t, each thread over a contiguous index range (index order)
-  const int span = (n + kStThreads - 1) / kStThreads;
-  const int b0 = min(n, t * span), b1 = min(n, b0 + span);
-  double eq = 0.0;
-  for (int i = b0; i < b1; ++i) eq += __float_as_uint(row[i]) == tk ? 1.0 : 0.0;
-  double rank = block_excl_scan(eq, 0.0, s_w);
-  __syncthreads();
-  const double keep_eq = tv > 0.0 ? fmax(1.0, ceil((static_cast<double>(top_p) - G) / tv)) : 1.0;
-  double kept = 0.0;
-  for (int i = b0; i < b1; ++i) {
-    const uint32_t k = __float_as_uint(row[i]);
-    bool keep = k > tk;
-    if (k == tk) {
-      keep = rank < keep_eq;
-      rank += 1.0;
+    for (int e = 0; e < kToppBatch; ++e) raw[e] = lr[min(i0 + e * kStThreads, a.n - 1)];
+#pragma unroll
+    for (int e = 0; e < kToppBatch; ++e) pin(raw[e]);
+#pragma unroll
+    for (int e = 0; e < kToppBatch; ++e) {
+      const float p = row_p(a, rs, raw[e]);
+      if (i0 + e * kStThreads < b1 && p != 0.f)
+        atomicAdd(&s_mass[topp_bin(__float_as_uint(p))], static_cast<double>(p));
     }
-    if (keep) kept += static_cast<double>(row[i]);
   }
-  // kept mass: per-thread sums in index order, then the threads in order
-  const double before = block_excl_scan(kept, 0.0, s_w);
   __syncthreads();
-  __shared__ double s_tot;
-  if (t == kStThreads - 1) s_tot = before + kept;
-  __syncthreads();
-  const double tot = s_tot;
-  rank = block_excl_scan(eq, 0.0, s_w);
-  for (int i = b0; i < b1; ++i) {
-    const float v = row[i];
-    const uint32_t k = __float_as_uint(v);
-    bool keep = k > tk;
-    if (k == tk) {
-      keep = rank < keep_eq;
-      rank += 1.0;
+  double* h = w.hist + (static_cast<int64_t>(r) * w.parts + blockIdx.x) * kWarpBins;
+  for (int b = t; b < kWarpBins; b += kStThreads) h[b] = s_mass[b];
+}
+
+__global__ __launch_bounds__(kStThreads) void k_topp_bound(WarpArgs w) {
+  const ProbsArgs& a = w.a;
+  const int t = threadIdx.x, r = blockIdx.y, per = (a.n + w.parts - 1) / w.parts;
+  const int b0 = blockIdx.x * per, b1 = min(a.n, b0 + per);
+  __shared__ RsShared sh;
+  __shared__ uint32_t s_bin;
+  __shared__ double s_above;
+  // the crossing bin: the row's masses, largest bins first (thread t: 8 bins down from kWarpBins - 1 - 8 t)
+  constexpr int PER = kWarpBins / kStThreads;
+  double m[PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) m[e] = 0.0;
+  for (int q = 0; q < w.parts; ++q) {
+    const double* h = w.hist + (static_cast<int64_t>(r) * w.parts + q) * kWarpBins;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) m[e] += h[kWarpBins - 1 - t * PER - e];
+  }
+  double own = 0.0;
+#pragma unroll
+  for (int e = 0; e < PER; ++e) own += m[e];
+  if (t == 0) s_bin = 0xffffffffu;
+  double c = block_excl_scan(own, 0.0, sh.w);
+  uint32_t low = 0xffffffffu;
+  double low_above = 0.0;
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {
+    const uint32_t b = kWarpBins - 1 - t * PER - e;
+    if (c < w.top_p && c + m[e] >= w.top_p) {
+      s_bin = b;
+      s_above = c;
     }
-    row[i] = keep ? static_cast<float>(static_cast<double>(v) / tot) : 0.f;
+    if (m[e] > 0.0) {
+      low = b;
+      low_above = c;
+    }
+    c += m[e];
+  }
+  __syncthreads();
+  if (s_bin == 0xffffffffu) {  // rounding left the target just past the row's mass: the lowest bin in use
+    __syncthreads();
+    if (t == 0) sh.digit[0] = 0xffffffffu;
+    __syncthreads();
+    if (low != 0xffffffffu) atomicMin(&sh.digit[0], low);
+    __syncthreads();
+    if (low == sh.digit[0] && low != 0xffffffffu) {
+      s_bin = low;
+      s_above = low_above;
+    }
+    if (t == 0 && sh.digit[0] == 0xffffffffu) {
+      s_bin = 0;
+      s_above = 0.0;
+    }
+    __syncthreads();
+  }
+  const uint32_t bin = s_bin;
+  const double above = s_above;
+  const RowSoftmax rs = row_softmax(a, r);
+  const float* lr = a.logits + static_cast<int64_t>(r) * a.ld;
+  unsigned int* count = w.count + r * kCounterStride;
+  unsigned long long* list = w.list + static_cast<int64_t>(r) * kWarpList;
+  for (int i0 = b0; i0 < b1; i0 += kStThreads * kToppBatch) {
+    float raw[kToppBatch];
+#pragma unroll
+    for (int e = 0; e < kToppBatch; ++e) raw[e] = lr[min(i0 + e * kStThreads + t, a.n - 1)];
+#pragma unroll
+    for (int e = 0; e < kToppBatch; ++e) pin(raw[e]);
+#pragma unroll
+    for (int e = 0; e < kToppBatch; ++e) {
+      const int i = i0 + e * kStThreads + t;
+      const uint32_t key = __float_as_uint(row_p(a, rs, raw[e]));
+      warp_append(i < b1 && key != 0 && topp_bin(key) == bin,
+                  static_cast<unsigned long long>(key) << 32 | static_cast<unsigned int>(i), count, list);
+    }
+  }
+  if (!warp_last(w.ctr + r * kCounterStride, gridDim.x)) return;
+  __shared__ unsigned long long s_list[kWarpList];
+  const int nc = static_cast<int>(__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  __syncthreads();
+  if (t == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  WarpSel sel;
+  if (nc <= kWarpList && nc > 0) {
+    for (int i = t; i < nc; i += kStThreads) s_list[i] = atomic_load_u64(list + i);
+    __syncthreads();
+    sel = topp_select([&](int i) { return __uint_as_float(static_cast<uint32_t>(s_list[i] >> 32)); },
+                      [&](int i) { return static_cast<int>(static_cast<uint32_t>(s_list[i])); }, nc, w.top_p, above,
+                      sh);
+  } else {  // a bin of more entries than the list holds (near-uniform rows): over the whole row
+    sel = topp_select([&](int i) { return row_p(a, rs, lr[i]); }, [](int i) { return i; }, a.n, w.top_p, 0.0, sh);
+  }
+  if (t == 0) w.sel[r] = sel;
+}
+
+__global__ __launch_bounds__(kStThreads) void k_topp_write(WarpArgs w) {
+  const ProbsArgs& a = w.a;
+  const int t = threadIdx.x, r = blockIdx.y, x0 = blockIdx.x * kVocabChunk;
+  const float* lr = a.logits + static_cast<int64_t>(r) * a.ld;
+  float* orow = a.out + static_cast<int64_t>(r) * a.ld_out;
+  float raw[kPerThread];
+#pragma unroll
+  for (int e = 0; e < kPerThread; ++e) raw[e] = lr[min(x0 + e * kStThreads + t, a.n - 1)];
+#pragma unroll
+  for (int e = 0; e < kPerThread; ++e) pin(raw[e]);
+  const WarpSel sel = w.sel[r];
+  const RowSoftmax rs = row_softmax(a, r);
+#pragma unroll
+  for (int e = 0; e < kPerThread; ++e) {
+    const int i = x0 + e * kStThreads + t;
+    const float p = row_p(a, rs, raw[e]);
+    const uint32_t key = __float_as_uint(p);
+    const bool keep = key > sel.key || (key == sel.key && i <= sel.last);
+    if (i < a.n) orow[i] = keep ? static_cast<float>(static_cast<double>(p) / sel.mass) : 0.f;
   }
 }
 
@@ -1949,9 +2608,15 @@ static int tree_stochastic(const float* p, int rows, int vocab, int64_t ld_p, co
   a.purpose = rng->purpose;
   a.st = reinterpret_cast<TreeState*>(static_cast<char*>(workspace) + kTreeStateOff);
   a.chunk_data = reinterpret_cast<double*>(static_cast<char*>(workspace) + kStochChunkOff);
+  a.sums = reinterpret_cast<double*>(static_cast<char*>(workspace) + kTreeSumsOff);
+  a.nodes = reinterpret_cast<TreeNode*>(static_cast<char*>(workspace) + kTreeNodesOff);
+  a.bad_parts = reinterpret_cast<int32_t*>(a.nodes + WC_MAX_NODES);
+  a.chunk_rows = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + kChunkRowsOff);
   a.counter = verify_counter(workspace, kCtrTree);
   a.verdict = verdict_dev;
   auto s = reinterpret_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(k_tree_sums, dim3(kTreeParts, rows), dim3(kStThreads), 0, s, a);
+  WC_LAUNCHED();
   hipLaunchKernelGGL(k_tree_walk, dim3(1), dim3(kTwThreads), 0, s, a);
   WC_LAUNCHED();
   hipLaunchKernelGGL(k_tree_sample, dim3((vocab + kVocabChunk - 1) / kVocabChunk), dim3(kStThreads), 0, s, a);
@@ -1985,13 +2650,52 @@ int wc_probs_from_logits(const float* logits, int rows, int n, int64_t ld, float
   a.ld_out = ld_out;
   a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + kProbsOff);
   a.kth_key = nullptr;
-  const dim3 grid((n + kVocabChunk - 1) / kVocabChunk, rows);
+  const int nch = (n + kVocabChunk - 1) / kVocabChunk;
+  const dim3 grid(nch, rows);
   auto s = reinterpret_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  WarpArgs w{};
+  w.a = a;
+  w.top_p = static_cast<double>(top_p);
+  w.ctr = reinterpret_cast<unsigned int*>(ws + kWarpCtrOff);
+  w.count = w.ctr + WC_MAX_NODES * kCounterStride;
+  w.maxima = reinterpret_cast<uint32_t*>(ws + kWarpMaxOff);
+  w.bound = reinterpret_cast<uint32_t*>(ws + kWarpOff);
+  w.list = reinterpret_cast<unsigned long long*>(ws + kWarpListOff);
+  w.hist = reinterpret_cast<double*>(ws + kWarpHistOff);
+  w.sel = reinterpret_cast<WarpSel*>(ws + kWarpSelOff);
   if (top_k > 0 && top_k < n) {  // sampling.py:41-43: x < the k-th largest x -> -inf
-    uint32_t* keys = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kWarpOff);
-    hipLaunchKernelGGL(k_topk_key, dim3(rows), dim3(kStThreads), 0, s, a, top_k, keys);
+    // about four blocks per CU, at least sixteen a row (60 rows of 151,936: 24 +
+    // 27 us; a block per chunk of 4,096 measured 27 + 25); group maxima: as
+    // many as fit the row's slots, and enough that their k-th largest is a close
+    // bound; the list's finishing block reads the row again where it overflows,
+    // so the output must not overlay the logits
+    w.k = top_k;
+    const int blocks = std::max(1, std::min(nch, std::max(16, 1024 / rows)));
+    w.span = ((n + blocks - 1) / blocks + 3) / 4 * 4;
+    const int used = (n + w.span - 1) / w.span;
+    w.groups = kStThreads;
+    while (w.groups > 4 && w.groups * used > kWarpGroups) w.groups /= 2;
+    const char *l0 = reinterpret_cast<const char*>(logits), *o0 = reinterpret_cast<const char*>(out);
+    const size_t lb = (static_cast<size_t>(rows - 1) * ld + n) * 4, ob = (static_cast<size_t>(rows - 1) * ld_out + n) * 4;
+    const bool apart = l0 + lb <= o0 || o0 + ob <= l0;
+    if (top_k <= kTopkMax && w.groups * used <= kWarpGroups && w.groups * used >= 4 * top_k && apart) {
+      const dim3 kgrid(used, rows);
+      if (n % 4 == 0 && ld % 4 == 0 && ld_out % 4 == 0 && aligned(logits, 16) && aligned(out, 16)) {
+        hipLaunchKernelGGL(k_topk_bound<true>, kgrid, dim3(kStThreads), 0, s, w);
+        WC_LAUNCHED();
+        hipLaunchKernelGGL(k_topk_finish<true>, kgrid, dim3(kStThreads), 0, s, w);
+      } else {
+        hipLaunchKernelGGL(k_topk_bound<false>, kgrid, dim3(kStThreads), 0, s, w);
+        WC_LAUNCHED();
+        hipLaunchKernelGGL(k_topk_finish<false>, kgrid, dim3(kStThreads), 0, s, w);
+      }
+      WC_LAUNCHED();
+      return WC_OK;
+    }
+    hipLaunchKernelGGL(k_topk_key, dim3(rows), dim3(kStThreads), 0, s, a, top_k, w.bound);
     WC_LAUNCHED();
-    a.kth_key = keys;
+    a.kth_key = w.a.kth_key = w.bound;
   }
   if (n <= kSrMax && top_p >= 1.f) {  // the draft head's width: one launch, a block per row
     hipLaunchKernelGGL(k_softmax_row, dim3(rows), dim3(kSrThreads), 0, s, a);
@@ -2000,12 +2704,19 @@ int wc_probs_from_logits(const float* logits, int rows, int n, int64_t ld, float
   }
   hipLaunchKernelGGL(k_softmax_part, grid, dim3(kStThreads), 0, s, a);
   WC_LAUNCHED();
-  hipLaunchKernelGGL(k_softmax_write, grid, dim3(kStThreads), 0, s, a);
-  WC_LAUNCHED();
-  if (top_p < 1.f) {  // sampling.py:45-54
-    hipLaunchKernelGGL(k_topp, dim3(rows), dim3(kStThreads), 0, s, a, top_p);
+  if (top_p >= 1.f) {
+    hipLaunchKernelGGL(k_softmax_write, grid, dim3(kStThreads), 0, s, a);
     WC_LAUNCHED();
+    return WC_OK;
   }
+  // sampling.py:45-54
+  w.parts = std::max(1, std::min(std::min(16, kWarpHists / rows), nch));
+  hipLaunchKernelGGL(k_topp_hist, dim3(w.parts, rows), dim3(kStThreads), 0, s, w);
+  WC_LAUNCHED();
+  hipLaunchKernelGGL(k_topp_bound, dim3(w.parts, rows), dim3(kStThreads), 0, s, w);
+  WC_LAUNCHED();
+  hipLaunchKernelGGL(k_topp_write, grid, dim3(kStThreads), 0, s, w);
+  WC_LAUNCHED();
   return WC_OK;
 }
 

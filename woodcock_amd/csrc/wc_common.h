@@ -334,7 +334,30 @@ constexpr size_t kWarpOff = kStochDecOff + kStochDecBytes;
 constexpr size_t kWarpBytes = 4 * WC_MAX_NODES;
 constexpr size_t kGridBarOff = kWarpOff + kWarpBytes;
 constexpr size_t kGridBarBytes = 2 * 8 * kMailSetWords + 128;
-constexpr size_t kVerifyWorkspace = kGridBarOff + kGridBarBytes;
+// warping over several blocks per row (wc_probs_from_logits): per row two
+// counters (blocks done, candidates listed) on lines of their own, the maxima of
+// kWarpGroups groups of entries, a list of kWarpList candidates, the top-p
+// result; and kWarpHists histograms of kWarpBins probability bins (fp64 masses)
+constexpr int kWarpGroups = 2048, kWarpList = 4096, kWarpBins = 2048, kWarpHists = 512;
+constexpr size_t kWarpCtrOff = (kGridBarOff + kGridBarBytes + 255) / 256 * 256;
+constexpr size_t kWarpCtrBytes = 2 * 4 * kCounterStride * static_cast<size_t>(WC_MAX_NODES);
+constexpr size_t kWarpMaxOff = kWarpCtrOff + kWarpCtrBytes;
+constexpr size_t kWarpMaxBytes = 4 * static_cast<size_t>(WC_MAX_NODES) * kWarpGroups;
+constexpr size_t kWarpListOff = kWarpMaxOff + kWarpMaxBytes;
+constexpr size_t kWarpListBytes = 8 * static_cast<size_t>(WC_MAX_NODES) * kWarpList;
+constexpr size_t kWarpSelOff = kWarpListOff + kWarpListBytes;
+constexpr size_t kWarpSelBytes = 16 * static_cast<size_t>(WC_MAX_NODES);
+constexpr size_t kWarpHistOff = kWarpSelOff + kWarpSelBytes;
+constexpr size_t kWarpHistBytes = 8 * static_cast<size_t>(kWarpHists) * kWarpBins;
+// stochastic trees: per node and part (draft mass, target mass on the head rows,
+// target mass), per node (head row, p and q of its token at its parent), and a
+// flag set by the blocks that found d2t invalid
+constexpr int kTreeParts = 16;
+constexpr size_t kTreeSumsOff = kWarpHistOff + kWarpHistBytes;
+constexpr size_t kTreeSumsBytes = 8 * 3 * static_cast<size_t>(kTreeParts) * WC_MAX_NODES;
+constexpr size_t kTreeNodesOff = kTreeSumsOff + kTreeSumsBytes;
+constexpr size_t kTreeNodesBytes = 16 * static_cast<size_t>(WC_MAX_NODES) + 4 * static_cast<size_t>(kTreeParts);
+constexpr size_t kVerifyWorkspace = (kTreeNodesOff + kTreeNodesBytes + 255) / 256 * 256;
 inline unsigned int* verify_counter(void* ws, int which) {
   return reinterpret_cast<unsigned int*>(static_cast<char*>(ws) + kCounterOff + which * kTreeCounterBytes);
 }
