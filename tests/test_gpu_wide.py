@@ -1,4 +1,5 @@
-"""Many-row passes (csrc/wide.hip) against the oracle: prompts through the
+"""Many-row passes (csrc/wide.hip) and the backend operations on them against
+the oracle and 64-bit torch: prompts through the
 drafter (fuse and forward) at the edges of the row tiles (16, 128) and of a pass
 (1024), few rows over a long context (the keys split over blocks), head sizes with and without the flash attention, both cache types, a
 sliding window, two layers.
@@ -95,3 +96,75 @@ def test_fuse_gathers_rows_and_bf16_taps(cuda, rows):
               ptr(got), 256, ptr(d.ws), stream_ptr())
     want = d.fuse([t[idx.long().clamp(0, 39)].float() for t in taps])
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("L,K,N", [(1, 8, 3), (1, 2056, 4100), (2, 520, 7), (3, 512, 33), (7, 4104, 129), (8, 64, 5000),
+                                   (9, 32, 1), (16, 96, 50), (17, 2048, 1030), (33, 544, 64), (65, 256, 8200),
+                                   (130, 2048, 2048), (600, 128, 6145)])
+def test_linear_shapes(cuda, wdt, L, K, N):
+    """Row counts around the vector / matrix-core boundary (8 | 9), odd widths and
+    outputs, tiles past the last row and column; sums in fp32 against 64 bits."""
+    from woodcock_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(L * K + N)
+    x = torch.randn(L, K, generator=g, device=cuda)
+    W = torch.randn(N, K, generator=g, device=cuda).to(wdt)
+    y0 = torch.randn(L, N, generator=g, device=cuda)
+    want = x.double() @ W.double().T
+    # |error| <= a few roundings of the largest partial sum, ~ sqrt(K) for unit inputs
+    tol = 8 * 2.0 ** -24 * K ** 0.5 * 4
+    pad = torch.full((L * N + 64,), 7.0, device=cuda)
+    y = pad[:L * N].view(L, N)
+    ops.linear(x, W, y=y)
+    assert (y.double() - want).abs().max() < tol * 4
+    assert (pad[L * N:] == 7).all()
+    acc = y0.clone()
+    ops.linear(x, W, y=acc, accumulate=True)
+    assert (acc.double() - (y0.double() + want)).abs().max() < tol * 5
+
+
+@pytest.mark.parametrize("L", [4, 40])
+def test_linear_infinities_and_nan(cuda, L):
+    """An infinite or NaN entry reaches exactly the outputs it reaches in fp32."""
+    from woodcock_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(L)
+    x = torch.randint(1, 4, (L, 64), generator=g, device=cuda).float()
+    W = torch.randint(1, 4, (96, 64), generator=g, device=cuda).bfloat16()
+    x[1, 5] = float("inf")
+    x[2, 7] = float("nan")
+    W[3, 9] = float("-inf")
+    got, want = ops.linear(x, W), (x.double() @ W.double().T).float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isnan(want).any()
+    assert torch.equal(got[~torch.isnan(want)], want[~torch.isnan(want)])
+
+
+@pytest.mark.parametrize("L,T,H,Hk,masked", [(1, 1, 4, 2, False), (1, 65, 8, 8, False), (3, 257, 4, 1, True),
+                                             (20, 33, 8, 2, True), (64, 64, 16, 8, True), (128, 129, 16, 8, True),
+                                             (200, 1000, 8, 4, True), (300, 70, 4, 4, False)])
+def test_attention_shapes(cuda, L, T, H, Hk, masked):
+    """Both head_dim 128 kernels around their limits, masks of unaligned row
+    lengths with rows that see one key only, values past the last key untouched."""
+    from woodcock_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(L * T)
+    q = torch.randn(L, H, 128, generator=g, device=cuda)
+    K = torch.randn(T + 3, Hk, 128, generator=g, device=cuda)
+    V = torch.randn(T + 3, Hk, 128, generator=g, device=cuda)
+    K[T:], V[T:] = float("nan"), float("nan")
+    K, V = K[:T], V[:T]
+    m = None
+    if masked:
+        m = torch.rand(L, T, generator=g, device=cuda) < 0.5
+        m[:, 0] |= ~m.any(dim=1)
+        m[0] = False
+        m[0, T - 1] = True
+    got = ops.attention(q, K, V, m, 0.09)
+    kd, vd = (t.double().transpose(0, 1).repeat_interleave(H // Hk, 0) for t in (K, V))
+    z = q.double().transpose(0, 1) @ kd.transpose(1, 2).contiguous() * 0.09
+    if m is not None:
+        z = z.masked_fill(~m[None], -float("inf"))
+    want = (torch.softmax(z, dim=2) @ vd).transpose(0, 1)
+    # weights of relative error ~ |z| 2^-23 (|z| < 6) against values of unit size
+    assert (got.double() - want).abs().max() < 1e-5

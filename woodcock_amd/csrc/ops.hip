@@ -12,9 +12,11 @@
 // off) where the reference rounds them separately.  Layouts are the reference's: activations
 // [rows][cols], the attention's K / V as its KVCache rows [T][Hk][D].
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "wc_common.h"
+#include "wide.h"
 
 namespace wc {
 
@@ -133,6 +135,7 @@ __global__ __launch_bounds__(kOpThreads) void k_op_softmax(float* x, int n) {
 
 // ------------------------------------------------------------------ attention
 
+// Other head sizes and alignments than the kernels below take.
 // block (query row l, head h): softmax(scale * q K^T + mask) V over T keys of kv
 // head h / (H / Hk), 256 keys per chunk with a running max; thread d < D owns
 // output element d.
@@ -212,6 +215,207 @@ __global__ __launch_bounds__(kOpThreads) void k_op_linear(const float* x, int L,
       *yp = accumulate ? *yp + v : v;
     }
   }
+}
+
+// Few rows (NL = 1, 2, 4 or 8 held by every wave): wave = R output rows, a lane 8
+// consecutive k of each 512-wide step by 16-byte loads, four steps in flight.
+// in a multiple of 8, x and W 16-byte aligned.
+template <int NL, int R, bool WF>
+__global__ __launch_bounds__(kOpThreads) void k_op_linear_vec(const float* x, int L, int in, const void* W, int out,
+                                                              float* y, int accumulate) {
+  constexpr int WV = WF ? 2 : 1;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int n0 = (blockIdx.x * (kOpThreads / kWave) + wave) * R;
+  if (n0 >= out) return;
+  float s[R][NL];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int l = 0; l < NL; ++l) s[r][l] = 0.f;
+  constexpr int U = NL * R <= 4 ? 4 : 2;  // steps in flight
+  for (int k0 = lane * 8; k0 < in; k0 += 512 * U) {
+    uint4 w[U][R][WV];
+    float4 xv[U][NL][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + u * 512, in - 8);  // (a step past the end re-reads the last values, unused)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int h = 0; h < WV; ++h)
+          w[u][r][h] = *reinterpret_cast<const uint4*>(static_cast<const char*>(W) +
+                                                       (static_cast<int64_t>(min(n0 + r, out - 1)) * in + k) * (WF ? 4 : 2) +
+                                                       16 * h);
+#pragma unroll
+      for (int l = 0; l < NL; ++l)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          xv[u][l][h] = *reinterpret_cast<const float4*>(x + static_cast<int64_t>(min(l, L - 1)) * in + k + 4 * h);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // (selects, not a branch: loads behind one would wait one after another)
+      const bool live = k0 + u * 512 < in;
+#pragma unroll
+      for (int l = 0; l < NL; ++l)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float4& v = xv[u][l][h];
+          v = float4{live ? v.x : 0.f, live ? v.y : 0.f, live ? v.z : 0.f, live ? v.w : 0.f};
+        }
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int h = 0; h < WV; ++h) {
+          uint4& v = w[u][r][h];
+          v = make_uint4(live ? v.x : 0u, live ? v.y : 0u, live ? v.z : 0u, live ? v.w : 0u);
+        }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float wv[8];
+        if constexpr (WF) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const uint4 q = w[u][r][e / 4];
+            wv[e] = __uint_as_float(e % 4 == 0 ? q.x : e % 4 == 1 ? q.y : e % 4 == 2 ? q.z : q.w);
+          }
+        } else {
+          const uint4 q = w[u][r][0];
+          wv[0] = bf16_lo(q.x); wv[1] = bf16_hi(q.x); wv[2] = bf16_lo(q.y); wv[3] = bf16_hi(q.y);
+          wv[4] = bf16_lo(q.z); wv[5] = bf16_hi(q.z); wv[6] = bf16_lo(q.w); wv[7] = bf16_hi(q.w);
+        }
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+          const float4 p = xv[u][l][0], q = xv[u][l][1];
+          float v = s[r][l];
+          v = fmaf(p.x, wv[0], v);
+          v = fmaf(p.y, wv[1], v);
+          v = fmaf(p.z, wv[2], v);
+          v = fmaf(p.w, wv[3], v);
+          v = fmaf(q.x, wv[4], v);
+          v = fmaf(q.y, wv[5], v);
+          v = fmaf(q.z, wv[6], v);
+          s[r][l] = fmaf(q.w, wv[7], v);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      const float v = wave_sum_dpp(s[r][l]);
+      if (lane == 0 && l < L && n0 + r < out) {
+        float* yp = y + static_cast<int64_t>(l) * out + n0 + r;
+        *yp = accumulate ? *yp + v : v;
+      }
+    }
+}
+
+template <int NL, bool WF>
+static void linear_vec_t(const float* x, int L, int in, const void* W, int out, float* y, int accumulate,
+                         hipStream_t s) {
+  // one output row per wave up to 4096 rows (1024 blocks), two beyond
+  constexpr int W4 = kOpThreads / kWave;
+  if (out <= 4096 || NL > 4)
+    hipLaunchKernelGGL((k_op_linear_vec<NL, 1, WF>), dim3((out + W4 - 1) / W4), dim3(kOpThreads), 0, s, x, L, in, W,
+                       out, y, accumulate);
+  else
+    hipLaunchKernelGGL((k_op_linear_vec<NL, 2, WF>), dim3((out + 2 * W4 - 1) / (2 * W4)), dim3(kOpThreads), 0, s, x, L,
+                       in, W, out, y, accumulate);
+}
+
+// ------------------------------------------------------------------ few-row attention
+
+// Block (row, head), head_dim 128: the 64 groups of 16 lanes take keys g, g + 64,
+// .. (8 dims per lane, 16-byte loads), each with its own running max, fp64 sum
+// and output; the groups merge in LDS.  K, V, q and out 16-byte aligned.
+constexpr int kOaThreads = 1024;
+constexpr int kOaGroups = kOaThreads / 16;
+__global__ __launch_bounds__(kOaThreads) void k_op_attention_vec(const float* q, int H, int Hk, const float* K,
+                                                                 const float* V, int T, const uint8_t* mask,
+                                                                 float* out, float scale) {
+  constexpr int D = 128, B = 4;  // keys in flight per group
+  __shared__ float s_o[kOaGroups][D + 4];
+  __shared__ float s_m[kOaGroups];
+  __shared__ double s_l[kOaGroups];
+  const int l = blockIdx.x, h = blockIdx.y, t = threadIdx.x, g = t / 16, d0 = t % 16 * 8;
+  const int kh = h / (H / Hk);
+  const int64_t kv_ld = static_cast<int64_t>(Hk) * D;
+  const float* qp = q + (static_cast<int64_t>(l) * H + h) * D + d0;
+  const float* kp = K + static_cast<int64_t>(kh) * D + d0;
+  const float* vp = V + static_cast<int64_t>(kh) * D + d0;
+  const uint8_t* mp = mask ? mask + static_cast<int64_t>(l) * T : nullptr;
+  const float4 qa = *reinterpret_cast<const float4*>(qp), qb = *reinterpret_cast<const float4*>(qp + 4);
+  float m = -INFINITY;
+  double ls = 0.0;
+  float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int j0 = g; j0 < T; j0 += kOaGroups * B) {
+    float4 ka[B], kb[B], va[B], vb[B];
+    uint32_t on[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int64_t at = static_cast<int64_t>(min(j0 + u * kOaGroups, T - 1)) * kv_ld;
+      ka[u] = *reinterpret_cast<const float4*>(kp + at);
+      kb[u] = *reinterpret_cast<const float4*>(kp + at + 4);
+      va[u] = *reinterpret_cast<const float4*>(vp + at);
+      vb[u] = *reinterpret_cast<const float4*>(vp + at + 4);
+      on[u] = mp ? mp[min(j0 + u * kOaGroups, T - 1)] : 1;
+    }
+    float sc[B], mx = m;
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      float dot = ka[u].x * qa.x;
+      dot = fmaf(ka[u].y, qa.y, dot);
+      dot = fmaf(ka[u].z, qa.z, dot);
+      dot = fmaf(ka[u].w, qa.w, dot);
+      dot = fmaf(kb[u].x, qb.x, dot);
+      dot = fmaf(kb[u].y, qb.y, dot);
+      dot = fmaf(kb[u].z, qb.z, dot);
+      dot = fmaf(kb[u].w, qb.w, dot);
+      dot = row16_sum(dot);
+      sc[u] = j0 + u * kOaGroups < T && on[u] ? __fmul_rn(scale, dot) : -INFINITY;
+      mx = fmaxf(mx, sc[u]);
+    }
+    const float al = mx == -INFINITY ? 1.f : expf(m - mx);
+    m = mx;
+    ls *= al;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= al;
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      // (a key past the end adds nothing: its value row is another key's)
+      const float p = sc[u] == -INFINITY ? 0.f : expf(sc[u] - m);
+      if (j0 + u * kOaGroups >= T) continue;
+      ls += static_cast<double>(p);
+      o[0] = fmaf(p, va[u].x, o[0]);
+      o[1] = fmaf(p, va[u].y, o[1]);
+      o[2] = fmaf(p, va[u].z, o[2]);
+      o[3] = fmaf(p, va[u].w, o[3]);
+      o[4] = fmaf(p, vb[u].x, o[4]);
+      o[5] = fmaf(p, vb[u].y, o[5]);
+      o[6] = fmaf(p, vb[u].z, o[6]);
+      o[7] = fmaf(p, vb[u].w, o[7]);
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s_o[g][d0 + e] = o[e];
+  if (t % 16 == 0) {
+    s_m[g] = m;
+    s_l[g] = ls;
+  }
+  __syncthreads();
+  if (t >= D) return;
+  float M = s_m[0];
+  for (int k = 1; k < kOaGroups; ++k) M = fmaxf(M, s_m[k]);
+  double L = 0.0;
+  float acc = 0.f;
+  for (int k = 0; k < kOaGroups; ++k) {
+    const float w = s_m[k] == -INFINITY ? 0.f : expf(s_m[k] - M);
+    L += s_l[k] * w;
+    acc = fmaf(s_o[k][t], w, acc);
+  }
+  out[(static_cast<int64_t>(l) * H + h) * D + t] = __fmul_rn(acc, static_cast<float>(1.0 / L));
 }
 
 // ------------------------------------------------------------------ KV cache rows
@@ -300,6 +504,41 @@ int wc_attention(const float* q, int L, int H, int Hk, int D, const float* K, co
              T, H, Hk);
   WC_REQUIRE(D >= 1 && D <= 256, "wc_attention: head_dim %d outside 1..256", D);
   if (L == 0) return WC_OK;
+  auto st = reinterpret_cast<hipStream_t>(stream);
+  if (D == 128 && aligned(q, 16) && aligned(K, 16) && aligned(V, 16) && aligned(out, 16)) {
+    // Times in us on 256 CUs: a round of the per-(row, head) blocks, two on a CU,
+    // against the 32-key chunks that a block of 64 query vectors walks.  1 row,
+    // 600 keys: 12 against 59 (33 on the general kernel); 64 rows, 1000 keys: 62
+    // / 102 (141); 128 rows, 128 keys: 53 / 17 (24); 384 rows, 1400 keys: 427 / 139
+    // (654).
+    int cus = 0;
+    if (int rc = device_cus(&cus)) return rc;
+    const int64_t blocks = static_cast<int64_t>(L) * H, rounds = (blocks + 2 * cus - 1) / (2 * cus);
+    const int64_t fblocks = (static_cast<int64_t>(L) * (H / Hk) + 63) / 64 * Hk;
+    const float per_row = rounds > 1 ? rounds * (12.f + .017f * T) : 6.f + .0115f * T;
+    const float flash = (fblocks + 2 * cus - 1) / (2 * cus) * (T / 32.f) * 3.2f + 4.f;
+    if (per_row <= flash) {
+      hipLaunchKernelGGL(k_op_attention_vec, dim3(L, H), dim3(kOaThreads), 0, st, q, H, Hk, K, V, T, mask, out, scale);
+      WC_LAUNCHED();
+      return WC_OK;
+    }
+    WideAttnArgs a{};
+    a.q = q;
+    a.ld_q = static_cast<int64_t>(H) * D;
+    a.H = H;
+    a.Hk = Hk;
+    a.rows = L;
+    a.k = K;
+    a.v = V;
+    a.ld_head = D;
+    a.ld_key = static_cast<int64_t>(Hk) * D;
+    a.keys = T;
+    a.mask = mask;
+    a.mask_ld = T;
+    a.scale = scale;
+    a.out = out;
+    return launch_wide_attn(a, WC_F32, st);
+  }
   hipLaunchKernelGGL(k_op_attention, dim3(L, H), dim3(kOpThreads), 0, reinterpret_cast<hipStream_t>(stream), q, H, Hk,
                      D, K, V, T, mask, out, scale);
   WC_LAUNCHED();
@@ -312,6 +551,30 @@ int wc_linear(const float* x, int L, int in, const void* W, int w_dtype, int out
   WC_REQUIRE(L >= 0 && in >= 1 && out >= 1, "wc_linear: bad shape L=%d in=%d out=%d", L, in, out);
   WC_REQUIRE(w_dtype == WC_F32 || w_dtype == WC_BF16, "wc_linear: weight dtype must be f32 or bf16");
   if (L == 0) return WC_OK;
+  if (in % 8 == 0 && aligned(x, 16) && aligned(W, 16)) {
+    auto st = reinterpret_cast<hipStream_t>(stream);
+    const bool wf = w_dtype == WC_F32;
+    // up to eight rows a wave holds them all (2048 x 2048 bf16: 1 row 18 -> 3.9 us,
+    // 8 rows 39 -> 9.2, 16 on the matrix cores); beyond, the matrix cores (16 rows
+    // 40 -> 17 us, 384 rows 840 -> 36)
+    if (L <= 8) {
+      auto go = [&](auto nl) {
+        constexpr int NL = decltype(nl)::value;
+        if (wf)
+          linear_vec_t<NL, true>(x, L, in, W, out, y, accumulate, st);
+        else
+          linear_vec_t<NL, false>(x, L, in, W, out, y, accumulate, st);
+      };
+      if (L == 1) go(std::integral_constant<int, 1>{});
+      else if (L == 2) go(std::integral_constant<int, 2>{});
+      else if (L <= 4) go(std::integral_constant<int, 4>{});
+      else go(std::integral_constant<int, 8>{});
+      WC_LAUNCHED();
+      return WC_OK;
+    }
+    if (in % 32 == 0) return launch_wide_linear(x, L, in, W, w_dtype, out, y, accumulate, st);
+  }
+  // other widths and alignments
   const dim3 grid((out + kOpThreads / kWave - 1) / (kOpThreads / kWave), (L + kLinRows - 1) / kLinRows);
   hipLaunchKernelGGL(k_op_linear, grid, dim3(kOpThreads), 0, reinterpret_cast<hipStream_t>(stream), x, L, in, W,
                      w_dtype, out, y, accumulate);

@@ -55,6 +55,11 @@ struct WideArgs {
 
 int launch_wide_gemm(const WideArgs& a, int epi, hipStream_t s);
 
+// y [L][out] (+)= x [L][in] . W [out][in]^T on the matrix cores: fp32 x, bf16 or
+// fp32 W, in a multiple of 32, x and W 16-byte aligned
+int launch_wide_linear(const float* x, int L, int in, const void* W, int w_dtype, int out, float* y, int accumulate,
+                       hipStream_t s);
+
 // ------------------------------------------------------------------ q / k norm, RoPE, append (head_dim 128)
 
 struct WideQkvArgs {

@@ -445,6 +445,219 @@ __global__ __launch_bounds__(WM* WN* WK* kWave) __attribute__((amdgpu_waves_per_
   }
 }
 
+// ------------------------------------------------------------------ linear
+
+// The same product straight from fp32 rows and row-major weights, for callers
+// without a workspace for planes: a block splits what it stages.  Block tile BM
+// x BN, WK groups of WM x WN waves on alternate k steps; two LDS buffers in
+// fragment order, the next step's values in registers while the current one is
+// multiplied.  fp32 weights (WF) are split as the rows are: six products per
+// pair of fragments, everything down to 2^-24 of the leading one.  Sums as in
+// k_wide_gemm.
+struct WideLinArgs {
+  const float* x;
+  const void* w;
+  int M, N, K;
+  float* y;
+  int accumulate;
+  int vec;  // rows of y keep 16-byte vectors whole
+};
+
+template <int BM, int BN, int WM, int WN, int WK, int WPE, bool WF>
+__global__ __launch_bounds__(WM* WN* WK* kWave) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void k_wide_linear(
+    WideLinArgs a, int mblocks) {
+  constexpr int GW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
+  constexpr int AR = BM / 16 / GW, WR = BN / 16 / GW, WP = WF ? 3 : 1;
+  constexpr int ACH = BM / 16 * 3, WCH = BN / 16 * WP, SV = WK * (ACH + WCH) * 64;
+  static_assert(AR * GW * 16 == BM && WR * GW * 16 == BN, "whole tiles per wave");
+  static_assert(WK == 1 || (WK - 1) * BM * BN * 4 <= 2 * SV * 16, "the groups' sums fit the buffers");
+  __shared__ wu32x4 s_buf[2 * SV];
+  const int t = threadIdx.x, lane = t % kWave;
+  const int wv = __builtin_amdgcn_readfirstlane(t / kWave), grp = wv / GW, wave = wv % GW;
+  int blk;
+  {
+    const int nb = gridDim.x, q = nb / 8, r = nb % 8, x = blockIdx.x % 8, i = blockIdx.x / 8;
+    blk = x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
+  }
+  const int m0 = (blk % mblocks) * BM, n0 = blk / mblocks * BN;
+  const int steps = a.K / 32, stages = (steps + WK - 1) / WK;
+  const int wm = wave / WN, wn = wave % WN;
+
+  // this lane's 8 values of a fragment: row l % 16, k 8 (l / 16) .. + 7 (rows past the last re-read it)
+  const float* xp[AR];
+#pragma unroll
+  for (int i = 0; i < AR; ++i)
+    xp[i] = a.x + static_cast<int64_t>(min(m0 + (wave * AR + i) * 16 + lane % 16, a.M - 1)) * a.K + 8 * (lane / 16);
+  const char* wp[WR];
+#pragma unroll
+  for (int i = 0; i < WR; ++i)
+    wp[i] = static_cast<const char*>(a.w) +
+            (static_cast<int64_t>(min(n0 + (wave * WR + i) * 16 + lane % 16, a.N - 1)) * a.K + 8 * (lane / 16)) *
+                (WF ? 4 : 2);
+  wu32x4 rx[AR][2], rw[WR][WF ? 2 : 1];
+  auto fetch = [&](int st) {
+    const int64_t k = static_cast<int64_t>(min(st * WK + grp, steps - 1)) * 32;
+#pragma unroll
+    for (int i = 0; i < AR; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) rx[i][h] = *reinterpret_cast<const wu32x4*>(xp[i] + k + 4 * h);
+#pragma unroll
+    for (int i = 0; i < WR; ++i)
+#pragma unroll
+      for (int h = 0; h < (WF ? 2 : 1); ++h)
+        rw[i][h] = *reinterpret_cast<const wu32x4*>(wp[i] + k * (WF ? 4 : 2) + 16 * h);
+  };
+  auto split = [&](const wu32x4* r, wu32x4* d) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(r[e / 4][e % 4]);
+    uint4 h, m, l;
+    wd_split8(v, h, m, l);
+    d[0] = __builtin_bit_cast(wu32x4, h);
+    d[64] = __builtin_bit_cast(wu32x4, m);
+    d[128] = __builtin_bit_cast(wu32x4, l);
+  };
+  auto put = [&](int b) {
+    wu32x4* d = s_buf + b * SV + grp * (ACH + WCH) * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < AR; ++i) split(rx[i], d + (wave * AR + i) * 192);
+#pragma unroll
+    for (int i = 0; i < WR; ++i) {
+      if constexpr (WF)
+        split(rw[i], d + (ACH + (wave * WR + i) * 3) * 64);
+      else
+        d[(ACH + wave * WR + i) * 64] = rw[i][0];
+    }
+  };
+
+  wf32x4 hi[TN][TM], lo[TN][TM], tot[TN][TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) hi[j][i] = lo[j][i] = tot[j][i] = wf32x4{0.f, 0.f, 0.f, 0.f};
+  fetch(0);
+  put(0);
+  lds_barrier();
+  for (int st = 0; st < stages; ++st) {
+    if (st + 1 < stages) fetch(st + 1);
+    if (WK == 1 || st * WK + grp < steps) {
+      const wu32x4* d = s_buf + (st & 1) * SV + grp * (ACH + WCH) * 64 + lane;
+      wbf16x8 wf[TN][WP];
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < WP; ++q) wf[j][q] = __builtin_bit_cast(wbf16x8, d[(ACH + (wn * TN + j) * WP + q) * 64]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        wbf16x8 xf[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) xf[p] = __builtin_bit_cast(wbf16x8, d[((wm * TM + i) * 3 + p) * 64]);
+#pragma unroll
+        for (int p = 2; p >= 0; --p)
+#pragma unroll
+          for (int q = (WP - 1 < 2 - p ? WP - 1 : 2 - p); q >= 0; --q)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+              wf32x4& c = p + q ? lo[j][i] : hi[j][i];
+              c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][q], xf[p], c, 0, 0, 0);
+            }
+      }
+    }
+    if ((st + 1) % kWideFlush == 0 || st + 1 == stages) {
+      mfma_settle();
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const wf32x4 u = tot[j][i] + hi[j][i];
+          lo[j][i] += hi[j][i] - (u - tot[j][i]);
+          tot[j][i] = u;
+          hi[j][i] = wf32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    if (st + 1 < stages) put((st + 1) & 1);
+    lds_barrier();
+  }
+  mfma_settle();
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i) tot[j][i] += lo[j][i];
+  if constexpr (WK > 1) {
+    float4* sum = reinterpret_cast<float4*>(s_buf);
+    if (grp > 0) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+          sum[((grp - 1) * GW + wave) * TN * TM * 64 + (j * TM + i) * 64 + lane] =
+              float4{tot[j][i][0], tot[j][i][1], tot[j][i][2], tot[j][i][3]};
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int g = 0; g < WK - 1; ++g)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const float4 v = sum[(g * GW + wave) * TN * TM * 64 + (j * TM + i) * 64 + lane];
+          tot[j][i] += wf32x4{v.x, v.y, v.z, v.w};
+        }
+  }
+
+  // An infinite input meets zero terms of the other operand, which leaves NaN
+  // where the product is infinite: a wave with such a sum takes plain fp32 sums
+  // of its tile instead.
+  bool odd = false;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(tot[j][i][e]) <= 3.402823466e38f);
+  if (__ballot(odd) != 0) {
+    for (int c = lane; c < TM * 16 * TN * 16; c += kWave) {
+      const int m = m0 + wm * TM * 16 + c / (TN * 16), n = n0 + wn * TN * 16 + c % (TN * 16);
+      if (m >= a.M || n >= a.N) continue;
+      const float* xr = a.x + static_cast<int64_t>(m) * a.K;
+      float v = 0.f;
+      for (int k = 0; k < a.K; ++k) {
+        const int64_t at = static_cast<int64_t>(n) * a.K + k;
+        v = fmaf(xr[k], WF ? static_cast<const float*>(a.w)[at] : bf16_to_float(static_cast<const uint16_t*>(a.w)[at]), v);
+      }
+      float* yp = a.y + static_cast<int64_t>(m) * a.N + n;
+      *yp = a.accumulate ? *yp + v : v;
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + (wm * TM + i) * 16 + lane % 16;
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + (wn * TN + j) * 16 + 4 * (lane / 16);
+      float* yp = a.y + static_cast<int64_t>(m) * a.N + n;
+      if (a.vec && n < a.N) {
+        float4 v{tot[j][i][0], tot[j][i][1], tot[j][i][2], tot[j][i][3]};
+        if (a.accumulate) {
+          const float4 q = *reinterpret_cast<const float4*>(yp);
+          v.x += q.x;
+          v.y += q.y;
+          v.z += q.z;
+          v.w += q.w;
+        }
+        *reinterpret_cast<float4*>(yp) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < a.N) yp[e] = a.accumulate ? yp[e] + tot[j][i][e] : tot[j][i][e];
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ q / k norm, RoPE, append
 
 // One wave per head vector of 128: lane j holds dims j and j + 64, a RoPE pair.
@@ -851,6 +1064,51 @@ int launch_wide_gemm(const WideArgs& a, int epi, hipStream_t s) {
     case 3: wide_gemm_t<64, 128, 2, 2, 1, 4, 2>(a, epi, s); break;
     case 4: wide_gemm_t<128, 128, 4, 2, 1, 4, 2>(a, epi, s); break;
     default: wide_gemm_t<128, 128, 2, 2, 1, 2, 2>(a, epi, s); break;
+  }
+  WC_LAUNCHED();
+  return WC_OK;
+}
+
+template <int BM, int BN, int WM, int WN, int WK, int WPE>
+static void wide_linear_t(const WideLinArgs& a, bool wf, hipStream_t s) {
+  const int mb = (a.M + BM - 1) / BM, nb = (a.N + BN - 1) / BN;
+  const dim3 grid(mb * nb), block(WM * WN * WK * kWave);
+  if (wf)
+    hipLaunchKernelGGL((k_wide_linear<BM, BN, WM, WN, WK, WPE, true>), grid, block, 0, s, a, mb);
+  else
+    hipLaunchKernelGGL((k_wide_linear<BM, BN, WM, WN, WK, WPE, false>), grid, block, 0, s, a, mb);
+}
+
+int launch_wide_linear(const float* x, int L, int in, const void* W, int w_dtype, int out, float* y, int accumulate,
+                       hipStream_t s) {
+  int cus = 0;
+  if (int rc = device_cus(&cus)) return rc;
+  const WideLinArgs a{x, W, L, out, in, y, accumulate, out % 4 == 0 && aligned(y, 16)};
+  const bool wf = w_dtype == WC_F32;
+  // as launch_wide_gemm: the least rounds x step time, bf16 / fp32 weights (us,
+  // in 2048: 16 rows 2048 outputs 17 / 24 with 32 x 32, 160 rows 23 / 36 with 32 x
+  // 64, 384 rows 36 / 53 with 64 x 64, 384 rows 6144 outputs 69 / 110 with 64 x
+  // 128; 128 x 128 was never the best)
+  constexpr WideTile kTiles[2][4] = {
+      {{32, 32, .26f, .265f}, {32, 64, .34f, .345f}, {64, 64, .54f, .555f}, {64, 128, .80f, .54f}},
+      {{32, 32, .38f, .386f}, {32, 64, .53f, .53f}, {64, 64, .78f, .78f}, {64, 128, 1.25f, .86f}}};
+  int best = 0;
+  float best_t = 0.f;
+  for (int i = 0; i < 4; ++i) {
+    const WideTile& t = kTiles[wf][i];
+    const int64_t blocks = static_cast<int64_t>((L + t.bm - 1) / t.bm) * ((out + t.bn - 1) / t.bn);
+    const int64_t rounds = (blocks + cus - 1) / cus;
+    const float us = rounds > 1 ? rounds * t.more : t.one;
+    if (i == 0 || us < best_t) {
+      best = i;
+      best_t = us;
+    }
+  }
+  switch (best) {
+    case 0: wide_linear_t<32, 32, 2, 1, 4, 2>(a, wf, s); break;
+    case 1: wide_linear_t<32, 64, 2, 1, 4, 2>(a, wf, s); break;
+    case 2: wide_linear_t<64, 64, 2, 2, 2, 2>(a, wf, s); break;
+    default: wide_linear_t<64, 128, 2, 2, 1, 2>(a, wf, s); break;
   }
   WC_LAUNCHED();
   return WC_OK;
