@@ -37,6 +37,8 @@
 // distribution.  Node counts are data-dependent there (a row with fewer nonzero
 // entries than draws yields fewer children), so they live in the state and the
 // host's launch shapes are upper bounds.
+#include <type_traits>
+
 #include "wc_common.h"
 
 namespace wc {
@@ -78,7 +80,8 @@ constexpr int kTdMaxNodes = 512;
 constexpr int kTdMaxWidth = 8;
 constexpr int kTdThreads = 256;
 
-constexpr int kTdParts = 16;  // blocks per frontier row in the expansion
+constexpr int kTdParts = 16;        // blocks per frontier row in the sampled expansion
+constexpr int kTdExpandParts = 64;  // waves per frontier row in the greedy one, at most
 
 struct TreeDraftState {
   double phat[kTdMaxNodes];
@@ -88,7 +91,7 @@ struct TreeDraftState {
   int32_t front[kTdMaxWidth];  // node ids of the current frontier, in frontier-row order
   // expansion: each part's top-width keys per frontier row, and a counter per
   // row (own 128-byte line; reset by the block that completes it)
-  unsigned long long cand[kTdMaxWidth][kTdParts][kTdMaxWidth];
+  unsigned long long cand[kTdMaxWidth][kTdExpandParts][kTdMaxWidth];
   unsigned int ctr[kTdMaxWidth][32];
   // sampled drafting (T > 0): the table's node count, the last expansion's
   // node range, the current frontier's row count and the draws granted so far
@@ -106,7 +109,7 @@ struct TreeDraftState {
   unsigned int lvl_ctr[32];
   // greedy expansion from the logits: per frontier row and part, the part's
   // maximum and its sum of exp(z - maximum) (two fp32 bit patterns)
-  unsigned long long zstat[kTdMaxWidth][kTdParts];
+  unsigned long long zstat[kTdMaxWidth][kTdExpandParts];
 };
 
 __device__ __forceinline__ unsigned int atomic_load_u32(const unsigned int* p) {
@@ -142,149 +145,179 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
   return b;
 }
 
-// Block r: the `width` largest (q, lowest row first) entries of q row r.  Each
-// thread keeps a sorted top-width list of its share of the row, read as
-// 16-byte vectors kTdVec at a time (all loads of a pass issued before the
-// first insert); `width` block-wide maxima then pop the winners in order.
+// Wave-wide maximum of u32 keys by DPP moves; every lane receives it.
+__device__ __forceinline__ uint32_t wave_max_u32_dpp(uint32_t v) {
+  auto mv = [](uint32_t x, auto ctrl, auto mask) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), decltype(ctrl)::value,
+                                                             decltype(mask)::value, 0xf, false));
+  };
+  using std::integral_constant;
+  const integral_constant<int, 0xf> all{};
+  v = max(v, mv(v, integral_constant<int, 0xB1>{}, all));   // quad_perm [1,0,3,2]
+  v = max(v, mv(v, integral_constant<int, 0x4E>{}, all));   // quad_perm [2,3,0,1]
+  v = max(v, mv(v, integral_constant<int, 0x124>{}, all));  // row_ror:4
+  v = max(v, mv(v, integral_constant<int, 0x128>{}, all));  // row_ror:8
+  v = max(v, mv(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{}));  // row_bcast:15
+  v = max(v, mv(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{}));  // row_bcast:31
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
+// The `width` largest of the wave's entries (order key k[e], 0 = none; row i[e]),
+// the lower row first on a tie: lane j receives the j-th (key 0 past the last).
+// The winners are taken out of k.
+template <int NE>
+__device__ __forceinline__ void wave_top(uint32_t (&k)[NE], const int (&i)[NE], int width, uint32_t& key, int& row) {
+  const int lane = threadIdx.x % kWave;
+  key = 0;
+  row = 0;
+  for (int j = 0; j < width; ++j) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) m = max(m, k[e]);
+    const uint32_t M = wave_max_u32_dpp(m);
+    if (M == 0) return;  // uniform
+    int im = 0x7fffffff;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) im = k[e] == M ? min(im, i[e]) : im;
+    const int I = 0x7fffffff - static_cast<int>(wave_max_u32_dpp(static_cast<uint32_t>(0x7fffffff - im)));
+    if (lane == j) {
+      key = M;
+      row = I;
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) k[e] = k[e] == M && i[e] == I ? 0u : k[e];
+  }
+}
+
+// Block (r, p), one wave: part p of q row r.  Its `width` largest entries
+// (lowest row first on a tie) chunk by chunk -- 16 entries per lane, the winners
+// of the chunks before among them -- go to the row's last wave, which selects
+// from every part's and writes the children, one lane each.  The waves meet no
+// barrier: at one wave a part needs neither block-wide maxima nor sorted lists
+// (256-thread parts of 1,024 rows with eight-entry lists took 14.8 us per level
+// at four rows of 16,384, half of it in the last block's chains of loads).
 // LOGITS: the row holds the head logits z and q = softmax(z) (T = 1) is never
 // written: softmax is monotone, so the top-width of q are the top-width of z
 // (same tie rule), and a child's q = exp(z - M) / S comes from the row's
 // maximum M and sum S = sum_p S_p exp(m_p - M), combined in part order by the
-// last part from each part's maximum m_p and sum S_p of exp(z - m_p).  The
-// exponential and the in-part sums follow k_softmax_row (expf; lane sums, the
-// wave sums, then the waves in order): only the association of the row sum
-// differs, a few ulps of q.
-constexpr int kTdVec = 8;
+// last wave from each part's maximum m_p and sum S_p of exp(z - m_p): against
+// k_softmax_row only the association of the row sum differs, a few ulps of q.
+constexpr int kTdChunk = 1024;
 template <bool LOGITS>
-__global__ __launch_bounds__(kTdThreads) void k_td_expand(TreeDraftState* st, const float* __restrict__ q,
-                                                          int head_rows, int64_t ld_q,
-                                                          const int32_t* __restrict__ d2t, int width,
-                                                          int node_base) {
-  __shared__ unsigned long long red[kTdThreads / kWave];
-  __shared__ float s_f[kTdThreads / kWave];
-  __shared__ float s_row[2];
-  __shared__ bool s_last;
-  const int r = blockIdx.x, p = blockIdx.y, P = gridDim.y, t = threadIdx.x;
+__global__ __launch_bounds__(kWave) void k_td_expand(TreeDraftState* st, const float* __restrict__ q, int head_rows,
+                                                     int64_t ld_q, const int32_t* __restrict__ d2t, int width,
+                                                     int node_base) {
+  constexpr int PER = kTdChunk / kWave;
+  __shared__ float s_part[kTdExpandParts];
+  const int r = blockIdx.x, p = blockIdx.y, P = gridDim.y, lane = threadIdx.x;
   const float* qr = q + static_cast<int64_t>(r) * ld_q;
   // part p: the rows [i0, i1) of the head (a multiple of 4 long, so aligned rows stay aligned)
   const int span = ((head_rows + P - 1) / P + 3) & ~3;
   const int i0 = min(p * span, head_rows), i1 = min(i0 + span, head_rows);
-  unsigned long long top[kTdMaxWidth];
+  const bool al = (reinterpret_cast<uintptr_t>(qr) & 15) == 0 && i1 % 4 == 0;
+  const int v = st->front[r];
+  // lane j: the part's j-th winner so far; the part's maximum and sum of exp
+  uint32_t wk = 0;
+  int wi = 0;
+  float mp = -INFINITY, sp = 0.f;
+  for (int c0 = i0; c0 < i1; c0 += kTdChunk) {
+    float z[PER];
+    uint32_t k[PER + 1];
+    int id[PER + 1];
+    if (al) {
+      float4 v4[PER / 4];
 #pragma unroll
-  for (int j = 0; j < kTdMaxWidth; ++j) top[j] = 0;
-  float mloc = -INFINITY;  // LOGITS: this thread's maximum
-  auto insert = [&](float v, int i) {
-    if constexpr (LOGITS) mloc = fmaxf(mloc, v);
-    unsigned long long k = argmax_key(v, i);
+      for (int u = 0; u < PER / 4; ++u)
+        v4[u] = *reinterpret_cast<const float4*>(qr + min(c0 + (u * kWave + lane) * 4, i1 - 4));
 #pragma unroll
-    for (int j = 0; j < kTdMaxWidth; ++j) {
-      const bool take = j < width && k > top[j];
-      const unsigned long long o = top[j];
-      top[j] = take ? k : o;
-      k = take ? o : k;
-    }
-  };
-  // 16-byte vectors where the row is 16-byte aligned, the tail (and unaligned rows) element-wise
-  const bool al = (reinterpret_cast<uintptr_t>(qr) & 15) == 0;
-  const int b4 = i0 / 4, e4 = al ? i1 / 4 : b4;
-  const float4* q4 = reinterpret_cast<const float4*>(qr);
-  for (int b = b4; b < e4; b += kTdThreads * kTdVec) {
-    float4 v[kTdVec];
-#pragma unroll
-    for (int u = 0; u < kTdVec; ++u) v[u] = q4[min(b + u * kTdThreads + t, e4 - 1)];
-#pragma unroll
-    for (int u = 0; u < kTdVec; ++u) {
-      const int i4 = b + u * kTdThreads + t;
-      if (i4 < e4) {
-        insert(v[u].x, 4 * i4);
-        insert(v[u].y, 4 * i4 + 1);
-        insert(v[u].z, 4 * i4 + 2);
-        insert(v[u].w, 4 * i4 + 3);
+      for (int u = 0; u < PER / 4; ++u) {
+        z[4 * u] = v4[u].x;
+        z[4 * u + 1] = v4[u].y;
+        z[4 * u + 2] = v4[u].z;
+        z[4 * u + 3] = v4[u].w;
       }
+    } else {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) z[e] = qr[min(c0 + (e / 4 * kWave + lane) * 4 + e % 4, i1 - 1)];
+#pragma unroll
+      for (int e = 0; e < PER; ++e) pin(z[e]);
     }
+    float m = mp;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      id[e] = c0 + (e / 4 * kWave + lane) * 4 + e % 4;
+      k[e] = id[e] < i1 ? float_order(z[e]) : 0u;
+      if (id[e] < i1) m = fmaxf(m, z[e]);
+    }
+    if constexpr (LOGITS) {
+      m = wave_max_dpp(m);
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) s += id[e] >= i1 || z[e] == -INFINITY ? 0.f : expf(z[e] - m);
+      s = wave_sum_dpp(s);
+      sp = mp == -INFINITY ? s : sp * expf(mp - m) + s;
+      mp = m;
+    }
+    k[PER] = wk;
+    id[PER] = wi;
+    wave_top(k, id, width, wk, wi);
   }
-  for (int i = 4 * e4 + t; i < i1; i += kTdThreads) insert(qr[i], i);
   if constexpr (LOGITS) {
-    // the part's maximum, then its sum of exp(z - maximum) over a second pass
-    // of the part (L2-resident after the first; a single pass with running
-    // sums rescaled at each new maximum measured slower)
-    const int lane = t % kWave, wave = t / kWave;
-    const float mw = wave_max_dpp(mloc);
-    if (lane == 0) s_f[wave] = mw;
-    __syncthreads();
-    float mp = s_f[0];
-#pragma unroll
-    for (int w = 1; w < kTdThreads / kWave; ++w) mp = fmaxf(mp, s_f[w]);
-    __syncthreads();
-    float sl = 0.f;
-    for (int i = i0 + t; i < i1; i += kTdThreads) {
-      const float v = qr[i];
-      sl += v == -INFINITY ? 0.f : expf(v - mp);
-    }
-    sl = wave_sum_dpp(sl);
-    if (lane == 0) s_f[wave] = sl;
-    __syncthreads();
-    float sp = 0.f;
-#pragma unroll
-    for (int w = 0; w < kTdThreads / kWave; ++w) sp += s_f[w];
-    if (t == 0)
+    if (lane == 0)
       atomic_store_u64(&st->zstat[r][p], (static_cast<unsigned long long>(__float_as_uint(mp)) << 32) |
                                              static_cast<unsigned long long>(__float_as_uint(sp)));
   }
-  // the part's top keys, largest first (keys are unique: the row is in the key)
-  for (int j = 0; j < width; ++j) {
-    const unsigned long long best = block_max_u64(top[0], red);
-    if (best != 0 && top[0] == best) {
-#pragma unroll
-      for (int i = 0; i + 1 < kTdMaxWidth; ++i) top[i] = top[i + 1];
-      top[kTdMaxWidth - 1] = 0;
-    }
-    if (t == 0) atomic_store_u64(&st->cand[r][p][j], best);
-  }
-  // the last part of the row to finish merges every part's keys
+  if (lane < width)
+    atomic_store_u64(&st->cand[r][p][lane],
+                     static_cast<unsigned long long>(wk) << 32 | static_cast<unsigned int>(wi));
+  // the row's last wave merges every part's winners
   __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (t == 0) {
-    const bool last = __hip_atomic_fetch_add(&st->ctr[r][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                      static_cast<unsigned int>(P - 1);
-    if (last) __hip_atomic_store(&st->ctr[r][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = last;
+  unsigned int seen = 0;
+  if (lane == 0) seen = __hip_atomic_fetch_add(&st->ctr[r][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  seen = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<int>(seen)));
+  if (seen != static_cast<unsigned int>(P - 1)) return;
+  if (lane == 0) __hip_atomic_store(&st->ctr[r][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  constexpr int NC = kTdExpandParts * kTdMaxWidth / kWave;
+  uint32_t k[NC];
+  int id[NC];
+  const int n = P * width;
+  unsigned long long c[NC];
+#pragma unroll
+  for (int e = 0; e < NC; ++e) {
+    const int x = min(e * kWave + lane, n - 1);
+    c[e] = e * kWave < n ? atomic_load_u64(&st->cand[r][x / width][x % width]) : 0ull;
   }
-  __syncthreads();
-  if (!s_last) return;
-  unsigned long long k = t < P * width ? atomic_load_u64(&st->cand[r][t / width][t % width]) : 0ull;
+  unsigned long long w = 0;
+  if constexpr (LOGITS) w = atomic_load_u64(&st->zstat[r][min(lane, P - 1)]);
+#pragma unroll
+  for (int e = 0; e < NC; ++e) {
+    k[e] = e * kWave + lane < n ? static_cast<uint32_t>(c[e] >> 32) : 0u;
+    id[e] = static_cast<int>(static_cast<uint32_t>(c[e]));
+  }
+  float M = 0.f, S = 1.f;
   if constexpr (LOGITS) {
-    if (t == 0) {
-      float mp[kTdParts], sp[kTdParts], M = -INFINITY;
-      for (int j = 0; j < P; ++j) {
-        const unsigned long long w = atomic_load_u64(&st->zstat[r][j]);
-        mp[j] = __uint_as_float(static_cast<uint32_t>(w >> 32));
-        sp[j] = __uint_as_float(static_cast<uint32_t>(w & 0xffffffffu));
-        M = fmaxf(M, mp[j]);
-      }
-      float S = 0.f;
-      for (int j = 0; j < P; ++j) S += sp[j] == 0.f ? 0.f : sp[j] * expf(mp[j] - M);
-      s_row[0] = M;
-      s_row[1] = S;
-    }
-    __syncthreads();
+    const float pm = lane < P ? __uint_as_float(static_cast<uint32_t>(w >> 32)) : -INFINITY;
+    const float ps = lane < P ? __uint_as_float(static_cast<uint32_t>(w)) : 0.f;
+    M = wave_max_dpp(pm);
+    s_part[lane] = ps == 0.f ? 0.f : ps * expf(pm - M);  // (one wave: no barrier)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    S = 0.f;
+    for (int j = 0; j < P; ++j) S += s_part[j];
   }
-  const int v = st->front[r];
-  for (int j = 0; j < width; ++j) {
-    const unsigned long long best = block_max_u64(k, red);
-    if (best != 0 && k == best) k = 0;
-    if (t == 0) {
-      const int row = argmax_key_index(best);
-      const int c = node_base + r * width + j;
-      st->token[c] = d2t ? d2t[row] : row;
-      st->parent[c] = v;
-      st->depth[c] = st->depth[v] + 1;
-      const float qc = LOGITS ? expf(qr[row] - s_row[0]) / s_row[1] : qr[row];
-      st->phat[c] = st->phat[v] * static_cast<double>(qc);
-      st->slot[c] = -1;
-      st->store[c] = -1;
-    }
-  }
+  uint32_t key;
+  int row;
+  wave_top(k, id, width, key, row);
+  if (lane >= width) return;
+  const int node = node_base + r * width + lane;
+  const float x = qr[row];
+  st->token[node] = d2t ? d2t[row] : row;
+  st->parent[node] = v;
+  st->depth[node] = st->depth[v] + 1;
+  st->phat[node] = st->phat[v] * static_cast<double>(LOGITS ? expf(x - M) / S : x);
+  st->slot[node] = -1;
+  st->store[node] = -1;
 }
 
 // One block: next frontier among the level's nodes [lb, le) and the inputs of
@@ -299,7 +332,14 @@ __global__ __launch_bounds__(kTdThreads) void k_td_frontier(TreeDraftState* st, 
   __shared__ int s_anc[kTdMaxWidth][kTdMaxNodes / kTdMaxWidth];
   __shared__ int s_nanc[kTdMaxWidth], s_pos[kTdMaxWidth];
   __shared__ double s_ph[kTdMaxNodes];
+  __shared__ int s_par[kTdMaxNodes], s_slot[kTdMaxNodes];
   const int t = threadIdx.x;
+  // the ancestor walks' tables, requested before anything waits
+#pragma unroll
+  for (int j = 0; j < kTdMaxNodes / kTdThreads; ++j) {
+    s_par[t + j * kTdThreads] = st->parent[t + j * kTdThreads];
+    s_slot[t + j * kTdThreads] = st->slot[t + j * kTdThreads];
+  }
   // level_begin 0: the level the last sampled expansion appended (its range is
   // in the state); rows [m, width) then get inputs of a harmless padding row
   const bool dyn = lb == 0;
@@ -314,6 +354,7 @@ __global__ __launch_bounds__(kTdThreads) void k_td_frontier(TreeDraftState* st, 
   for (int i = t; i < n; i += kTdThreads) {
     const double ph = s_ph[i];
     int rank = 0;
+#pragma unroll 8
     for (int u = 0; u < n; ++u) {
       const double pu = s_ph[u];
       rank += (pu > ph || (pu == ph && u < i)) ? 1 : 0;
@@ -327,13 +368,13 @@ __global__ __launch_bounds__(kTdThreads) void k_td_frontier(TreeDraftState* st, 
     const int v = s_front[t];
     st->front[t] = v;
     tokens[t] = st->token[v];
-    feat_rows[t] = st->store[st->parent[v]];
+    feat_rows[t] = st->store[s_par[v]];
     s_pos[t] = positions[t] = base - 1 + st->depth[v];
     st->slot[v] = base + tree_cache + t;
     st->store[v] = store_base + t;
     // cache slots of the ancestors below the root
     int na = 0;
-    for (int u = st->parent[v]; u > 0 && na < kTdMaxNodes / kTdMaxWidth; u = st->parent[u]) s_anc[t][na++] = st->slot[u];
+    for (int u = s_par[v]; u > 0 && na < kTdMaxNodes / kTdMaxWidth; u = s_par[u]) s_anc[t][na++] = s_slot[u];
     s_nanc[t] = na;
   } else if (t < rows) {  // padding: the root token on the root's feedback at depth 1, seeing the prefix and itself
     tokens[t] = st->token[0];
@@ -376,6 +417,7 @@ __global__ __launch_bounds__(kTdThreads) void k_td_select(const TreeDraftState* 
       const double ph = s_ph[v];
       const int dv = s_dep[v];
       int rank = 0;
+#pragma unroll 8
       for (int u = 1; u < n_nodes; ++u) {
         const double pu = s_ph[u];
         const int du = s_dep[u];
@@ -839,9 +881,8 @@ int wc_tree_draft_expand(void* state, const float* q, int rows, int head_rows, i
   WC_REQUIRE(node_base >= 1 && node_base + rows * width <= kTdMaxNodes,
              "wc_tree_draft_expand: nodes %d..%d outside the table of %d", node_base, node_base + rows * width,
              kTdMaxNodes);
-  // parts of at least 1024 head rows each, at most kTdParts per frontier row
-  const int parts = std::max(1, std::min(kTdParts, head_rows / 1024));
-  hipLaunchKernelGGL(k_td_expand<false>, dim3(rows, parts), dim3(kTdThreads), 0,
+  const int parts = std::max(1, std::min(kTdExpandParts, (head_rows + kTdChunk - 1) / kTdChunk));
+  hipLaunchKernelGGL(k_td_expand<false>, dim3(rows, parts), dim3(kWave), 0,
                      reinterpret_cast<hipStream_t>(stream), static_cast<TreeDraftState*>(state), q, head_rows, ld_q,
                      d2t_dev, width, node_base);
   WC_LAUNCHED();
@@ -859,8 +900,8 @@ int wc_tree_draft_expand_logits(void* state, const float* logits, int rows, int 
   WC_REQUIRE(node_base >= 1 && node_base + rows * width <= kTdMaxNodes,
              "wc_tree_draft_expand_logits: nodes %d..%d outside the table of %d", node_base, node_base + rows * width,
              kTdMaxNodes);
-  const int parts = std::max(1, std::min(kTdParts, head_rows / 1024));
-  hipLaunchKernelGGL(k_td_expand<true>, dim3(rows, parts), dim3(kTdThreads), 0,
+  const int parts = std::max(1, std::min(kTdExpandParts, (head_rows + kTdChunk - 1) / kTdChunk));
+  hipLaunchKernelGGL(k_td_expand<true>, dim3(rows, parts), dim3(kWave), 0,
                      reinterpret_cast<hipStream_t>(stream), static_cast<TreeDraftState*>(state), logits, head_rows, ld,
                      d2t_dev, width, node_base);
   WC_LAUNCHED();
