@@ -292,3 +292,54 @@ def test_expand_from_logits_equals_softmax_then_expand(cuda, head_rows):
         assert (x == y).all()
     assert np.abs(pb - pa).max() <= 1e-6 * np.abs(pa).max()
     assert np.all(pa[1:] > 0) and np.all(pa[1:] < 1)
+
+
+@pytest.mark.parametrize("logits", [False, True])
+@pytest.mark.parametrize("head_rows", [4, 1023, 1025, 2050, 65537, 151936])
+def test_expand_over_part_edges_with_ties(cuda, head_rows, logits):
+    """Both greedy expansions against a host sort over head sizes around the
+    1,024-row parts (one short part; a second part of a few rows; unaligned
+    rows; more than 64 parts' worth, so a part runs several chunks), with many
+    equal entries (the lowest row wins) and -inf logits.  The tokens are exact;
+    q = exp(z - M) / S in fp32 from up to 64 x 3 partial sums of at most 1,024
+    terms each (16 per lane, then six halving steps): |error| <= (16 + 6 + 64 +
+    3 + 8) ulps of 2^-24 relative = 6e-6."""
+    from woodcock_amd import _lib
+    from woodcock_amd.runtime import ptr, stream_ptr
+
+    width, off = 4, 40
+    rng = np.random.default_rng(head_rows)
+    x = np.round(rng.standard_normal((1 + width, head_rows)) * 4) / 4  # few distinct values
+    if logits:
+        x[:, rng.random(head_rows) < 0.3] = -np.inf
+        x[:, [0, head_rows // 2, head_rows - 1]] = [1.0, 1.25, 1.25]
+        x[:, 1] = np.where(np.isinf(x[:, 1]), -2.0, x[:, 1])
+    else:
+        x = np.exp(x) / 64
+    x = x.astype(np.float32)
+    z = torch.from_numpy(x).to(cuda)
+    st = torch.zeros(int(_lib.lib().wc_tree_draft_state_bytes()), dtype=torch.uint8, device=cuda)
+    root = torch.tensor([7], dtype=torch.int32, device=cuda)
+    offset = torch.tensor([off], dtype=torch.int32, device=cuda)
+    tok, feat, pos = (torch.empty(width, dtype=torch.int32, device=cuda) for _ in range(3))
+    mask = torch.empty(width, 64, dtype=torch.uint8, device=cuda)
+    entry = "wc_tree_draft_expand_logits" if logits else "wc_tree_draft_expand"
+    s = stream_ptr()
+    _lib.call("wc_tree_draft_begin", ptr(st), ptr(root), s)
+    _lib.call(entry, ptr(st), ptr(z), 1, head_rows, head_rows, None, width, 1, s)
+    _lib.call("wc_tree_draft_frontier", ptr(st), 1, 1 + width, width, ptr(offset), 0, 0, 1, ptr(tok), ptr(feat),
+              ptr(pos), ptr(mask), mask.stride(0), s)
+    _lib.call(entry, ptr(st), ptr(z[1:]), width, head_rows, head_rows, None, width, 1 + width, s)
+    torch.cuda.synchronize()
+    raw = st.cpu().numpy()
+    phat = raw[:8 * 512].view(np.float64)
+    token, parent, depth = (raw[8 * 512 + 4 * 512 * i:8 * 512 + 4 * 512 * (i + 1)].view(np.int32) for i in range(3))
+    for r in range(1 + width):
+        v = x[r].astype(np.float64)
+        q = np.exp(v - v.max()) / np.exp(v - v.max()).sum() if logits else v
+        best = np.lexsort((np.arange(head_rows), -v))[:width]
+        nodes = 1 + width * r + np.arange(width)
+        assert (token[nodes] == best).all()
+        assert (parent[nodes] == r).all() and (depth[nodes] == (1 if r == 0 else 2)).all()
+        want = (1.0 if r == 0 else phat[r]) * q[best]
+        assert np.abs(phat[nodes] - want).max() <= 6e-6 * want.max()
