@@ -56,7 +56,7 @@ typedef struct wc_verdict {
   int32_t n_uniforms;  /* uniforms consumed (stochastic rules), 0 for greedy */
   int32_t status;      /* 0; WC_E_INVALID when the device saw an invalid input; WC_E_HIP when a bounded wait gave up */
   int32_t reserved[3];
-  int32_t tokens[WC_MAX_NODES + 1]; /* accepted tokens then `next` (n_keep entries) */
+  int32_t tokens[WC_MAX_NODES + 1]; /* accepted tokens then `next` (n_keep entries; the greedy chain rule zeroes the rest) */
   int32_t keep[WC_MAX_NODES + 1];   /* verify-block rows kept: 0 then the accepted nodes */
 } wc_verdict;
 

@@ -144,6 +144,7 @@ _SIGS = {
 }
 
 _lib = None
+_fns: dict[str, C._CFuncPtr] = {}  # the library's entry points, bound once
 
 
 class WoodcockHipError(RuntimeError):
@@ -162,6 +163,7 @@ def lib() -> C.CDLL:
             fn = getattr(handle, name)
             fn.argtypes = args
             fn.restype = res
+            _fns[name] = fn
         v = handle.wc_version()
         if v != ABI_VERSION:
             raise WoodcockHipError(f"{LIB_PATH} has ABI {v}, expected {ABI_VERSION}: rebuild it")
@@ -183,7 +185,11 @@ def check(status: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    if _lib is None:
+        lib()
+    status = _fns[name](*args)
+    if status != WC_OK:
+        check(status)
 
 
 def stream_handle(stream=None) -> int | None:

@@ -90,7 +90,12 @@ __device__ __forceinline__ void verify_finish(int lane, unsigned long long* __re
       verdict->n_keep = a + 1;
       verdict->n_uniforms = 0;
       verdict->status = 0;
+      for (int i = 0; i < 3; ++i) verdict->reserved[i] = 0;
     }
+    // the entries past the path are zeros whatever the buffer held: a fresh
+    // verdict needs no fill launch before the verify
+    if (c > a) verdict->tokens[c] = verdict->keep[c] = 0;
+    if (c == kWave - 1) verdict->tokens[c + 1] = verdict->keep[c + 1] = 0;
   } else if (mode == kModeTree) {
     const int N = rows;
     const int tok = c < N ? tree_tokens[c] : -1;

@@ -62,6 +62,7 @@ class Drafter:
         n = int(_lib.lib().wc_drafter_workspace_bytes(C.byref(self.dims)))
         self.ws = torch.empty((n + 255) // 256 * 256, dtype=torch.uint8, device=dev)
         _lib.call("wc_workspace_init", ptr(self.ws), self.ws.numel(), stream_ptr())
+        self._zero = torch.zeros(1, dtype=torch.int32, device=dev)  # offset base of calls with a host-side offset
 
     # ------------------------------------------------------------------ setup
 
@@ -189,7 +190,6 @@ class Drafter:
         self._ensure_rope(cap + 64)
         dev = self.device
         tok = tok.to(dev, torch.int32)
-        ints = torch.tensor([offset], dtype=torch.int32).to(dev)
         pos = None
         if positions is not None:
             pos = torch.as_tensor(positions).reshape(-1).to(dev, torch.int32)
@@ -211,7 +211,7 @@ class Drafter:
         vp = (C.c_void_p * len(cache))(*[c.values.data_ptr() for c in cache])
         kvdt = _BF16 if cache[0].keys.dtype == torch.bfloat16 else _F32
         _lib.call("wc_drafter_forward", C.byref(self.dims), C.byref(self.wstruct), ptr(tok), ptr(f), f.stride(0),
-                  None, 0, L, None, kp, vp, kvdt, cap, ptr(ints), 0, ptr(pos), ptr(m), mask_ld, ptr(hid), ptr(out),
+                  None, 0, L, None, kp, vp, kvdt, cap, ptr(self._zero), int(offset), ptr(pos), ptr(m), mask_ld, ptr(hid), ptr(out),
                   None, ptr(self.ws), stream_ptr())
         for c in cache:
             c.offset = offset + L

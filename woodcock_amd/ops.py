@@ -17,17 +17,26 @@ from .runtime import device_of, ptr, stream_ptr
 
 
 def _f32(t: torch.Tensor, name: str) -> torch.Tensor:
-    device_of(t)
+    if not t.is_cuda:
+        device_of(t)
     if t.dtype != torch.float32 or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous float32 device tensor")
     return t
 
 
 def _weight(w: torch.Tensor, name: str):
-    device_of(w)
+    if not w.is_cuda:
+        device_of(w)
     if w.dtype not in (torch.float32, torch.bfloat16) or not w.is_contiguous():
         raise ValueError(f"{name} must be a contiguous float32 or bfloat16 device tensor")
     return _lib.WC_BF16 if w.dtype == torch.bfloat16 else _lib.WC_F32
+
+
+def _as(t: torch.Tensor, like: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """t contiguous on like's device in `dtype`; t itself when it is."""
+    if t.dtype is dtype and t.device == like.device and t.is_contiguous():
+        return t
+    return t.to(like.device, dtype).contiguous()
 
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -69,7 +78,7 @@ def rope(x: torch.Tensor, positions: torch.Tensor, base: float, table: tuple[tor
     if x.dim() != 3:
         raise ValueError("x must be [L, heads, head_dim]")
     L, heads, D = x.shape
-    pos = positions.to(x.device, torch.int32).contiguous()
+    pos = _as(positions, x, torch.int32)
     if pos.numel() != L:
         raise ValueError("one position per row")
     cos = sin = None
@@ -105,7 +114,7 @@ def attention(q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, mask: torch.Ten
         raise ValueError("K / V must be [T, Hk, head_dim] like q's head_dim")
     m = None
     if mask is not None:
-        m = mask.to(q.device, torch.uint8).contiguous()
+        m = _as(mask, q, torch.uint8)
         if m.shape != (L, T):
             raise ValueError(f"mask must be [{L}, {T}]")
     out = torch.empty_like(q)

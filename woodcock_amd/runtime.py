@@ -13,33 +13,45 @@ from . import _lib
 
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
+# A short call is bound by what the host does before the launch (the greedy
+# verify of 5 rows: 7 us of kernel under 16 us per call), so the plumbing of
+# every call stays off torch's Stream and device objects and ctypes' wrappers:
+# handles are plain ints (None for the null stream).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # absent in a torch built without a GPU
+
 
 def device_of(t: torch.Tensor) -> torch.device:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"expected a GPU tensor, got a tensor on {t.device}")
     return t.device
 
 
-def stream_ptr(stream: torch.cuda.Stream | None = None):
-    s = torch.cuda.current_stream() if stream is None else stream
-    return C.c_void_p(s.cuda_stream) if s.cuda_stream else None
+def _current_stream(index: int) -> int:
+    """The current stream's handle on device `index` of the calling thread."""
+    return torch.cuda.current_stream(index).cuda_stream if _raw_stream is None else _raw_stream(index)
+
+
+def stream_ptr(stream: torch.cuda.Stream | None = None) -> int | None:
+    if stream is not None:
+        return stream.cuda_stream or None
+    return _current_stream(torch.cuda.current_device()) or None
 
 
 def workspace(device: torch.device, stream: torch.cuda.Stream | None = None) -> torch.Tensor:
     """Zero-initialised verify workspace for (device, stream); kernels leave it zeroed."""
-    s = torch.cuda.current_stream(device) if stream is None else stream
-    key = (device.index if device.index is not None else torch.cuda.current_device(), s.cuda_stream)
-    ws = _workspaces.get(key)
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    s = _current_stream(index) if stream is None else stream.cuda_stream
+    ws = _workspaces.get((index, s))
     if ws is None:
         n = int(_lib.lib().wc_workspace_bytes())
         ws = torch.empty((n + 255) // 256 * 256, dtype=torch.uint8, device=device)
-        _lib.call("wc_workspace_init", ptr(ws), ws.numel(), stream_ptr(s))
-        _workspaces[key] = ws
+        _lib.call("wc_workspace_init", ptr(ws), ws.numel(), s or None)
+        _workspaces[(index, s)] = ws
     return ws
 
 
-def ptr(t: torch.Tensor | None):
-    return None if t is None else C.c_void_p(t.data_ptr())
+def ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def i32(x, device) -> torch.Tensor:
@@ -63,7 +75,7 @@ def reset_workspaces(device: torch.device | None = None) -> None:
     idx = None if device is None else (device.index if device.index is not None else torch.cuda.current_device())
     for (d, s), ws in _workspaces.items():
         if idx is None or d == idx:
-            _lib.call("wc_workspace_init", ptr(ws), ws.numel(), C.c_void_p(s) if s else None)
+            _lib.call("wc_workspace_init", ptr(ws), ws.numel(), s or None)
 
 
 def check_verdict(out: _lib.Verdict, ws: torch.Tensor | None = None) -> _lib.Verdict:

@@ -114,7 +114,8 @@ def verify_chain_greedy_dev(target_logits: torch.Tensor, draft_tokens: torch.Ten
     rows = lg.shape[0]
     if draft_tokens.numel() != rows - 1:
         raise ValueError(f"{rows} logit rows need {rows - 1} draft tokens, got {draft_tokens.numel()}")
-    verdict = new_verdict(lg.device) if verdict is None else verdict
+    if verdict is None:  # the greedy chain rule writes every entry: no fill launch before it
+        verdict = torch.empty(_lib.VERDICT_INTS, dtype=torch.int32, device=lg.device)
     _lib.call("wc_verify_chain_greedy", ptr(lg), rows, lg.shape[1], lg.stride(0), ptr(draft_tokens), ptr(verdict),
               ptr(workspace(lg.device)), stream_ptr())
     return verdict
