@@ -450,6 +450,8 @@ static bool launch_gemvf(const GemvArgs& a, hipStream_t s) {
 
 // Few-row VALU GEMV (k_gemvk, csrc/gemvk.hip): false when the launch does not fit it.
 bool launch_gemvk_any(const GemvArgs& a, bool pair, int xb, hipStream_t s);
+// Few-row gate / up pair, one block per CU (k_gemv_pair, csrc/gemvp.hip): false when the launch does not fit it.
+bool launch_gemv_pair(const GemvArgs& a, hipStream_t s);
 
 template <bool PAIR, int NIN, int XB>
 static bool launch_gemvx(const GemvArgs& a, int steps, hipStream_t s) {
@@ -497,8 +499,8 @@ static int launch_gemv(const GemvArgs& a, int /*R hint*/, hipStream_t s) {
   const bool pair = a.epi == kEpiSiluPair;
   bool done = false;
   if (a.wfrag) {
-    // fragment-major gate / up pair: the few-row MFMA kernel only
-    if (pair && a.n_in == 1 && xb == 0 && a.M > 1) done = launch_gemvf<true, 1, 0>(a, s);
+    // fragment-major gate / up pair: the few-row MFMA kernels only
+    if (pair && a.n_in == 1 && xb == 0 && a.M > 1) done = launch_gemv_pair(a, s) || launch_gemvf<true, 1, 0>(a, s);
     if (!done) return set_error(WC_E_UNSUPPORTED, "gemv: fragment-major weights need the few-row gate / up pair");
     WC_LAUNCHED();
     return WC_OK;
@@ -506,7 +508,7 @@ static int launch_gemv(const GemvArgs& a, int /*R hint*/, hipStream_t s) {
   if (a.M > 1 && a.M <= 8 && !a.few_mfma) done = launch_gemvk_any(a, pair, xb, s);
   if (!done && a.M > 1) {
     if (pair && a.n_in == 1 && xb == 0)
-      done = launch_gemvf<true, 1, 0>(a, s);
+      done = launch_gemv_pair(a, s) || launch_gemvf<true, 1, 0>(a, s);
     else if (!pair && a.n_in == 1 && xb == 0)
       done = launch_gemvf<false, 1, 0>(a, s);
     else if (!pair && a.n_in == 2 && xb == 2)
