@@ -390,7 +390,8 @@ static bool launch_gemvf(const GemvArgs& a, hipStream_t s) {
     bool ok = true;
     for (int i = 0; i < a.n_in; ++i) ok = ok && a.in[i].K <= 10240;
     // one-tile projections only: the gate / up pair and two-tile grids
-    // measured faster on k_gemvf (50 MB gate / up at M = 5: 14.2 against 17 us)
+    // measured faster on k_gemvf (50 MB gate / up at M = 5: 14.2 against 17 us;
+    // k_gemv_pair takes most pairs before they reach here)
     if (ok && !wide) {
       if constexpr (!PAIR) {
         if (gb == kAll) {
@@ -423,8 +424,9 @@ static bool launch_gemvf(const GemvArgs& a, hipStream_t s) {
   if constexpr (PAIR && NIN == 1) {
     if (a.wfrag) {
       if (gb != kAll) return false;
-      // four waves of four k steps in flight: 15.1 us for the Qwen3-1.7B pair at
-      // 5 rows (eight waves 14.8, sixteen 18.1; 17.0 on the row-major layout)
+      // (pairs k_gemv_pair does not take: K above 2560, few or very many
+      // features) four waves of four k steps in flight: 15.1 us for a 2048 x
+      // 6144 pair at 5 rows (eight waves 14.8, sixteen 18.1)
       if (stg && gf_stage_ok(reinterpret_cast<const void*>(&k_gemvf<2, 4, 4, PAIR, NIN, XB, kAll, true, true>),
                              WC_GF_DYN(2, 4)))
         hipLaunchKernelGGL((k_gemvf<2, 4, 4, PAIR, NIN, XB, kAll, true, true>), grid, dim3(4 * kWave),
