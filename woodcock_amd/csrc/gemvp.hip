@@ -44,7 +44,7 @@ __device__ __forceinline__ void gp_split3(const float* x, gpbf16x8 (&p)[3]) {
 // its last step's addresses and count as zeros).
 template <int NT, int PER, bool FRAG>
 __global__ __launch_bounds__(kGpWaves * kWave) void k_gemv_pair(GemvArgs a) {
-  constexpr int SL = PER > 8 ? (NT < 2 ? NT : 2) : (NT < 3 ? NT : 3);  // half tiles in flight
+  constexpr int SL = PER > 8 || (PER > 4 && NT > 3) ? (NT < 2 ? NT : 2) : (NT < 3 ? NT : 3);  // half tiles in flight
   __shared__ float s_c[kGpWaves][NT][4][kWave];
   __shared__ float s_ss[kGpWaves][kWave];
   __shared__ float s_inv[16];
@@ -105,19 +105,22 @@ __global__ __launch_bounds__(kGpWaves * kWave) void k_gemv_pair(GemvArgs a) {
   }
   s_ss[wave][lane] = ss;
 
-  gpf32x4 acc[NT];
+  // the leading terms and the two small ones in chains of their own: fewer
+  // roundings at the sum's size, and two chains in flight
+  gpf32x4 acc[NT], acl[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    acc[j] = gpf32x4{0.f, 0.f, 0.f, 0.f};
+    acc[j] = acl[j] = gpf32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
       // a repeated step: zero weights too (an infinite one times the zero input would be NaN)
       const uint32_t on = i0 + u < i1 ? 0xffffffffu : 0u;
       uint4 q = w[j % SL][u];
       q = make_uint4(q.x & on, q.y & on, q.z & on, q.w & on);
-#pragma unroll
-      for (int p = 0; p < 3; ++p)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gpbf16x8, q), xs[u][p], acc[j], 0, 0, 0);
+      const gpbf16x8 qb = __builtin_bit_cast(gpbf16x8, q);
+      acl[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qb, xs[u][2], acl[j], 0, 0, 0);
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qb, xs[u][0], acc[j], 0, 0, 0);
+      acl[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qb, xs[u][1], acl[j], 0, 0, 0);
     }
     if (j + SL < NT) issue(j % SL, j + SL);
   }
@@ -125,7 +128,7 @@ __global__ __launch_bounds__(kGpWaves * kWave) void k_gemv_pair(GemvArgs a) {
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s_c[wave][j][e][lane] = acc[j][e];
+    for (int e = 0; e < 4; ++e) s_c[wave][j][e][lane] = acc[j][e] + acl[j][e];
   __syncthreads();
   if (t < 16) {
     float tot = 0.f;
