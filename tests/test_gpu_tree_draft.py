@@ -343,3 +343,47 @@ def test_expand_over_part_edges_with_ties(cuda, head_rows, logits):
         assert (parent[nodes] == r).all() and (depth[nodes] == (1 if r == 0 else 2)).all()
         want = (1.0 if r == 0 else phat[r]) * q[best]
         assert np.abs(phat[nodes] - want).max() <= 6e-6 * want.max()
+
+
+@pytest.mark.parametrize("mask_ld", [61, 64])
+@pytest.mark.parametrize("window", [0, 20])
+def test_frontier_mask_over_row_strides(cuda, mask_ld, window):
+    """The second frontier's inputs with mask rows that are and are not 16-byte
+    aligned (one store per 16 columns or per column): the prefix inside the
+    window, the ancestor's slot and the row itself, every other byte zero."""
+    from woodcock_amd import _lib
+    from woodcock_amd.runtime import ptr, stream_ptr
+
+    width, off, head_rows = 4, 40, 2050
+    z = torch.from_numpy(np.random.default_rng(mask_ld).standard_normal((1 + width, head_rows)).astype(np.float32)).to(cuda)
+    st = torch.zeros(int(_lib.lib().wc_tree_draft_state_bytes()), dtype=torch.uint8, device=cuda)
+    root = torch.tensor([7], dtype=torch.int32, device=cuda)
+    offset = torch.tensor([off], dtype=torch.int32, device=cuda)
+    tok, feat, pos = (torch.empty(width, dtype=torch.int32, device=cuda) for _ in range(3))
+    mask = torch.full((width, mask_ld), 9, dtype=torch.uint8, device=cuda)
+    s = stream_ptr()
+
+    def frontier(lb, le, tree_cache, store):
+        _lib.call("wc_tree_draft_frontier", ptr(st), lb, le, width, ptr(offset), tree_cache, window, store, ptr(tok),
+                  ptr(feat), ptr(pos), ptr(mask), mask_ld, s)
+
+    _lib.call("wc_tree_draft_begin", ptr(st), ptr(root), s)
+    _lib.call("wc_tree_draft_expand_logits", ptr(st), ptr(z), 1, head_rows, head_rows, None, width, 1, s)
+    frontier(1, 1 + width, 0, 1)
+    _lib.call("wc_tree_draft_expand_logits", ptr(st), ptr(z[1:]), width, head_rows, head_rows, None, width, 1 + width, s)
+    frontier(1 + width, 1 + width + width * width, width, 1 + width)
+    torch.cuda.synchronize()
+    raw = st.cpu().numpy()
+    phat = raw[:8 * 512].view(np.float64)
+    token, parent = (raw[8 * 512 + 4 * 512 * i:8 * 512 + 4 * 512 * (i + 1)].view(np.int32) for i in range(2))
+    nodes = np.arange(1 + width, 1 + width + width * width)
+    front = nodes[np.lexsort((nodes, -phat[nodes]))[:width]]
+    want = np.zeros((width, mask_ld), np.uint8)
+    lo = max(0, off + 1 - window + 1) if window else 0
+    want[:, lo:off] = 1
+    want[np.arange(width), off + parent[front] - 1] = 1
+    want[np.arange(width), off + width + np.arange(width)] = 1
+    assert (mask.cpu().numpy() == want).all()
+    assert (tok.cpu().numpy() == token[front]).all()
+    assert (feat.cpu().numpy() == parent[front]).all()  # the parents' rows: 1 + frontier row
+    assert (pos.cpu().numpy() == off + 1).all()

@@ -333,44 +333,51 @@ __global__ __launch_bounds__(kTdThreads) void k_td_frontier(TreeDraftState* st, 
   __shared__ int s_anc[kTdMaxWidth][kTdMaxNodes / kTdMaxWidth];
   __shared__ int s_nanc[kTdMaxWidth], s_pos[kTdMaxWidth];
   __shared__ double s_ph[kTdMaxNodes];
-  __shared__ int s_par[kTdMaxNodes], s_slot[kTdMaxNodes];
+  __shared__ int s_par[kTdMaxNodes], s_slot[kTdMaxNodes], s_tok[kTdMaxNodes], s_dep[kTdMaxNodes], s_sto[kTdMaxNodes];
   const int t = threadIdx.x;
-  // the ancestor walks' tables, requested before anything waits
+  // The launch is a chain of loads of what other CUs just wrote, so the whole
+  // node table comes in one round trip (read as it was chosen from, the
+  // probabilities, then the chosen nodes, then their parents: 7.3 us, 4.3 now; entries
+  // past the nodes are never used).
+  const int base = *offset_dev;
+  const int dyn_lb = st->lvl_begin, dyn_le = st->lvl_end;
 #pragma unroll
   for (int j = 0; j < kTdMaxNodes / kTdThreads; ++j) {
-    s_par[t + j * kTdThreads] = st->parent[t + j * kTdThreads];
-    s_slot[t + j * kTdThreads] = st->slot[t + j * kTdThreads];
+    const int v = t + j * kTdThreads;
+    s_ph[v] = st->phat[v];
+    s_par[v] = st->parent[v];
+    s_slot[v] = st->slot[v];
+    s_tok[v] = st->token[v];
+    s_dep[v] = st->depth[v];
+    s_sto[v] = st->store[v];
   }
   // level_begin 0: the level the last sampled expansion appended (its range is
   // in the state); rows [m, width) then get inputs of a harmless padding row
   const bool dyn = lb == 0;
   if (dyn) {
-    lb = st->lvl_begin;
-    le = st->lvl_end;
+    lb = dyn_lb;
+    le = dyn_le;
   }
-  const int n = min(max(le - lb, 0), kTdMaxNodes), m = min(width, n);
+  const int n = min(max(le - lb, 0), kTdMaxNodes - lb), m = min(width, n);
   const int rows = dyn ? width : m;
-  for (int i = t; i < n; i += kTdThreads) s_ph[i] = st->phat[lb + i];
   __syncthreads();
   for (int i = t; i < n; i += kTdThreads) {
-    const double ph = s_ph[i];
+    const double ph = s_ph[lb + i];
     int rank = 0;
-#pragma unroll 8
     for (int u = 0; u < n; ++u) {
-      const double pu = s_ph[u];
+      const double pu = s_ph[lb + u];
       rank += (pu > ph || (pu == ph && u < i)) ? 1 : 0;
     }
     if (rank < m) s_front[rank] = lb + i;
   }
   __syncthreads();
-  const int base = *offset_dev;
   if (t == 0) st->n_front = m;
   if (t < m) {
     const int v = s_front[t];
     st->front[t] = v;
-    tokens[t] = st->token[v];
-    feat_rows[t] = st->store[s_par[v]];
-    s_pos[t] = positions[t] = base - 1 + st->depth[v];
+    tokens[t] = s_tok[v];
+    feat_rows[t] = s_sto[s_par[v]];
+    s_pos[t] = positions[t] = base - 1 + s_dep[v];
     st->slot[v] = base + tree_cache + t;
     st->store[v] = store_base + t;
     // cache slots of the ancestors below the root
@@ -378,21 +385,45 @@ __global__ __launch_bounds__(kTdThreads) void k_td_frontier(TreeDraftState* st, 
     for (int u = s_par[v]; u > 0 && na < kTdMaxNodes / kTdMaxWidth; u = s_par[u]) s_anc[t][na++] = s_slot[u];
     s_nanc[t] = na;
   } else if (t < rows) {  // padding: the root token on the root's feedback at depth 1, seeing the prefix and itself
-    tokens[t] = st->token[0];
+    tokens[t] = s_tok[0];
     feat_rows[t] = 0;
     s_pos[t] = positions[t] = base;
     s_nanc[t] = 0;
   }
   __syncthreads();
+  // the prefix, 16 columns per store where the rows allow, then the ancestors
+  // and the row itself
+  if ((reinterpret_cast<uintptr_t>(mask) & 15) == 0 && mask_ld % 16 == 0) {
+    for (int r = 0; r < rows; ++r) {
+      const int lo = window > 0 ? max(0, s_pos[r] - window + 1) : 0;
+      uint4* row = reinterpret_cast<uint4*>(mask + static_cast<int64_t>(r) * mask_ld);
+      for (int64_t c = t; c < mask_ld / 16; c += kTdThreads) {
+        uint32_t w[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          w[q] = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int64_t col = c * 16 + q * 4 + e;
+            w[q] |= (col >= lo && col < base ? 1u : 0u) << (8 * e);
+          }
+        }
+        row[c] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+    }
+  } else {
+    for (int r = 0; r < rows; ++r) {
+      const int lo = window > 0 ? max(0, s_pos[r] - window + 1) : 0;
+      uint8_t* row = mask + static_cast<int64_t>(r) * mask_ld;
+      for (int64_t c = t; c < mask_ld; c += kTdThreads) row[c] = c >= lo && c < base ? 1 : 0;
+    }
+  }
+  __syncthreads();  // the bytes below lie in the words above
   for (int r = 0; r < rows; ++r) {
-    const int pos = s_pos[r];
-    const int lo = window > 0 ? max(0, pos - window + 1) : 0;
-    const int self = base + tree_cache + r, na = s_nanc[r];
-    uint8_t* row = mask + static_cast<int64_t>(r) * mask_ld;
-    for (int64_t c = t; c < mask_ld; c += kTdThreads) {
-      bool on = (c >= lo && c < base) || c == self;
-      for (int k = 0; k < na; ++k) on = on || c == s_anc[r][k];
-      row[c] = on ? 1 : 0;
+    const int na = s_nanc[r];
+    if (t <= na) {
+      const int64_t c = t < na ? s_anc[r][t] : base + tree_cache + r;
+      if (c >= 0 && c < mask_ld) mask[static_cast<int64_t>(r) * mask_ld + c] = 1;
     }
   }
 }
@@ -407,26 +438,36 @@ __global__ __launch_bounds__(kTdThreads) void k_td_select(const TreeDraftState* 
   __shared__ int s_grp[kTdMaxNodes / kWave];  // kept nodes per 64-node group
   const int t = threadIdx.x, lane = t % kWave;
   const bool all = n_nodes - 1 <= budget;
-  for (int v = t; v < n_nodes; v += kTdThreads) {
+  // the node table in one round trip (entries past the nodes are never used):
+  // 5.9 us for 85 nodes, 10.8 with the chosen nodes read after the scan and one
+  // lane per node ranking
+  int tok[kTdMaxNodes / kTdThreads], par[kTdMaxNodes / kTdThreads];
+#pragma unroll
+  for (int j = 0; j < kTdMaxNodes / kTdThreads; ++j) {
+    const int v = t + j * kTdThreads;
     s_ph[v] = st->phat[v];
     s_dep[v] = st->depth[v];
+    tok[j] = st->token[v];
+    par[j] = st->parent[v];
   }
   __syncthreads();
-  for (int v = t; v < n_nodes; v += kTdThreads) {
-    bool keep = v == 0 || all;
-    if (!keep) {
-      const double ph = s_ph[v];
-      const int dv = s_dep[v];
-      int rank = 0;
-#pragma unroll 8
-      for (int u = 1; u < n_nodes; ++u) {
+  // four lanes rank a node against every fourth node each: 85 nodes take 44
+  // steps of the serial loop instead of 84
+  for (int v0 = 0; v0 < n_nodes; v0 += kTdThreads / 4) {
+    const int v = min(v0 + t / 4, n_nodes - 1);
+    const double ph = s_ph[v];
+    const int dv = s_dep[v];
+    int rank = 0;
+    if (!all)
+#pragma unroll 4
+      for (int u = 1 + t % 4; u < n_nodes; u += 4) {
         const double pu = s_ph[u];
         const int du = s_dep[u];
         rank += (pu > ph || (pu == ph && (du < dv || (du == dv && u < v)))) ? 1 : 0;
       }
-      keep = rank < budget;
-    }
-    s_pos[v] = keep ? 1 : 0;
+    rank += __shfl_xor(rank, 1);
+    rank += __shfl_xor(rank, 2);
+    if (t % 4 == 0 && v0 + t / 4 < n_nodes) s_pos[v] = v == 0 || all || rank < budget ? 1 : 0;
   }
   __syncthreads();
   // exclusive scan of the keep flags in node order, -1 marking a dropped node:
@@ -454,13 +495,13 @@ __global__ __launch_bounds__(kTdThreads) void k_td_select(const TreeDraftState* 
     *count = k;
   }
   __syncthreads();
-  for (int v = t; v < n_nodes; v += kTdThreads) {
-    const int i = s_pos[v];
+#pragma unroll
+  for (int j = 0; j < kTdMaxNodes / kTdThreads; ++j) {
+    const int v = t + j * kTdThreads, i = v < n_nodes ? s_pos[v] : -1;
     if (i < 0) continue;
-    const int p = st->parent[v];
-    tokens[i] = st->token[v];
-    depth[i] = st->depth[v];
-    parents[i] = p < 0 ? -1 : s_pos[p];
+    tokens[i] = tok[j];
+    depth[i] = s_dep[v];
+    parents[i] = par[j] < 0 ? -1 : s_pos[par[j]];
   }
 }
 
