@@ -196,3 +196,26 @@ def test_fragment_major_weight_layout(cuda, rows, cols):
     a = w.view(torch.int16).cpu().numpy().reshape(rows // 16, 16, cols // 32, 4, 8)
     want = a.transpose(0, 2, 3, 1, 4).reshape(-1)  # [T][s][g][i][e]: lane l = 16 g + i
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("inter,M", [(8448, 3), (9728, 17), (12288, 33), (9728, 60), (8448, 64)])
+def test_target_layer_wide_intermediate(cuda, inter, M):
+    """Intermediate sizes whose gate / up pair runs in blocks of six tiles (48
+    features; 9728 leaves the last block 32), at each row tile count.  With a
+    zero o_proj the layer adds the MLP of x alone, so the cache's rounding stays
+    out: the file's 2e-5 of an fp32 cache against 64 bits."""
+    cfg = TargetConfig(hidden_size=512, num_heads=4, num_kv_heads=2, head_dim=128, intermediate_size=inter)
+    w = random_layer(cfg, seed=inter + M, device=cuda)
+    w["self_attn.o_proj.weight"].zero_()
+    layer = TargetLayer(cfg, w, cuda)
+    cache = KVCache(cfg.num_kv_heads, cfg.head_dim, 128, torch.bfloat16, cuda)
+    x = torch.randn(M, cfg.hidden_size, generator=torch.Generator(device=cuda).manual_seed(M), device=cuda)
+    off = torch.tensor([0], dtype=torch.int32, device=cuda)
+    mask = torch.ones(M, M, dtype=torch.uint8, device=cuda)
+    got = layer(x.clone(), cache, off, positions=None, mask=mask).cpu().double() - x.cpu().double()
+    wd = {k: v.cpu().double() for k, v in w.items()}
+    xd = x.cpu().double()
+    h = xd * torch.rsqrt((xd * xd).mean(1, keepdim=True) + cfg.rms_norm_eps) * wd["post_attention_layernorm.weight"]
+    act = torch.nn.functional.silu(h @ wd["mlp.gate_proj.weight"].T) * (h @ wd["mlp.up_proj.weight"].T)
+    want = act @ wd["mlp.down_proj.weight"].T
+    assert norm_err(got.numpy(), want.numpy()) < 2e-5

@@ -645,10 +645,12 @@ __device__ __forceinline__ void sk_fix_last(const SkArgs& a, int cb, float* s_c,
 // activations), and no fix-up launch follows.
 // FTW > 0 (MT = 1): the fix-up of column ranges of 64 FTW runs in this launch
 // (sk_fix_last), with the QKV head epilogue when FQKV.
-template <int MT, bool PE = false, int FTW = 0, bool FQKV = false>
+// G: column tiles per block (even; other than kMwG with PE only).
+template <int MT, bool PE = false, int FTW = 0, bool FQKV = false, int G = kMwG>
 __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
   static_assert(FTW == 0 || (MT == 1 && !PE), "the fix-up in the GEMM takes one row tile");
-  constexpr int G = kMwG, FB = 16 * G, LDR = FB + 4;
+  static_assert(G == kMwG || (PE && G % 2 == 0), "gate / up tile pairs");
+  constexpr int FB = 16 * G, LDR = FB + 4;
   typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) float s_red[4][64 * LDR];
   const int t = threadIdx.x, lane = t % kWave;
@@ -737,8 +739,8 @@ __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
   __syncthreads();
   if constexpr (PE) {
     // four waves summed in order into wave 0's tile, then the pair epilogue
-    // of thread (row m, 8 act features from g * 8): gate at column
-    // 32 (f / 16) + f % 16 of the tile, up 16 columns further
+    // of thread (row m, 8 act features from g * 8, then 32 further): gate at
+    // column 32 (f / 16) + f % 16 of the tile, up 16 columns further
     for (int e = t * 4; e < a.M * FB; e += 256 * 4) {
       const int r = e / FB, c = e % FB;
       float4 v = *reinterpret_cast<const float4*>(&s_red[0][r * LDR + c]);
@@ -753,28 +755,31 @@ __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
       *reinterpret_cast<float4*>(&s_red[0][r * LDR + c]) = v;
     }
     __shared__ float s_inv[64];
-    const int m = t / 4, g = t % 4;
+    const int m = t / 4, g0 = t % 4;
     float tot = 0.f;
 #pragma unroll
     for (int q = 0; q < kSsMax; ++q) tot += ssv[q];
     tot += __shfl_xor(tot, 1);
     tot += __shfl_xor(tot, 2);
-    if (g == 0) s_inv[m] = a.ss ? 1.f / sqrtf(tot / static_cast<float>(a.ss_k) + a.eps) : 1.f;
+    if (g0 == 0) s_inv[m] = a.ss ? 1.f / sqrtf(tot / static_cast<float>(a.ss_k) + a.eps) : 1.f;
     __syncthreads();
     if (m >= a.M) return;
     const float inv = s_inv[m];
-    float z[8];
+    for (int g = g0; g < G; g += 4) {
+      const int n0 = cg * (G * 8) + g * 8;
+      if (n0 >= a.N / 2) break;  // (a last block with fewer features)
+      float z[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int f = g * 8 + e, gc = (f / 16) * 32 + f % 16;
-      const float gv = s_red[0][m * LDR + gc] * inv, uv = s_red[0][m * LDR + gc + 16] * inv;
-      z[e] = gv / (1.f + expf(-gv)) * uv;
+      for (int e = 0; e < 8; ++e) {
+        const int f = g * 8 + e, gc = (f / 16) * 32 + f % 16;
+        const float gv = s_red[0][m * LDR + gc] * inv, uv = s_red[0][m * LDR + gc + 16] * inv;
+        z[e] = gv / (1.f + expf(-gv)) * uv;
+      }
+      uint4 hi, lo;
+      split8(z, hi, lo);
+      *reinterpret_cast<uint4*>(a.xa_next + xa_index(m, n0, 0)) = hi;
+      *reinterpret_cast<uint4*>(a.xa_next + xa_index(m, n0, 1)) = lo;
     }
-    const int n0 = (cg >> 1) * 64 + (cg & 1) * 32 + g * 8;
-    uint4 hi, lo;
-    split8(z, hi, lo);
-    *reinterpret_cast<uint4*>(a.xa_next + xa_index(m, n0, 0)) = hi;
-    *reinterpret_cast<uint4*>(a.xa_next + xa_index(m, n0, 1)) = lo;
     return;
   }
   // four waves summed in order; rows < M as this split's partial
@@ -921,13 +926,29 @@ static int launch_wave(SkArgs g, int fix_tw, hipStream_t s) {
   if (g.epi == kSkSiluPair && fix_tw == 2 && g.xa_next && !g.out && g.N / (16 * kMwG) >= 128 &&
       g.n_ss <= 4 * kSsMax) {
     g.ks = 1;
-    const dim3 grid1(g.N / (16 * kMwG), 1);
+    // blocks of four tiles; of six where that many would put a second block on
+    // some of the 256 CUs, which then set the launch's end, and six put one on
+    // each at most: 2 x 9728 x 2560 at 60 rows 33.1 us in 304 blocks, 22.4 in
+    // 203 (4.4 TB/s).  At 192 blocks of four (2 x 6144 features) six would
+    // leave half of the CUs idle.
+    constexpr int kCus = 256;
+    const int n4 = g.N / (16 * kMwG), n6 = (g.N + 95) / 96;
+    const bool six = n4 > kCus && n6 <= kCus;
+    const dim3 grid1(six ? n6 : n4, 1);
+#define WC_MWP(MT)                                                                                \
+  do {                                                                                            \
+    if (six)                                                                                      \
+      hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 6>), grid1, dim3(256), 0, s, g);          \
+    else                                                                                          \
+      hipLaunchKernelGGL((k_mm_wave<MT, true>), grid1, dim3(256), 0, s, g);                       \
+  } while (0)
     switch ((g.M + 15) / 16) {
-      case 1: hipLaunchKernelGGL((k_mm_wave<1, true>), grid1, dim3(256), 0, s, g); break;
-      case 2: hipLaunchKernelGGL((k_mm_wave<2, true>), grid1, dim3(256), 0, s, g); break;
-      case 3: hipLaunchKernelGGL((k_mm_wave<3, true>), grid1, dim3(256), 0, s, g); break;
-      default: hipLaunchKernelGGL((k_mm_wave<4, true>), grid1, dim3(256), 0, s, g); break;
+      case 1: WC_MWP(1); break;
+      case 2: WC_MWP(2); break;
+      case 3: WC_MWP(3); break;
+      default: WC_MWP(4); break;
     }
+#undef WC_MWP
     WC_LAUNCHED();
     return WC_OK;
   }
