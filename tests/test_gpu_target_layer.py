@@ -198,10 +198,12 @@ def test_fragment_major_weight_layout(cuda, rows, cols):
     np.testing.assert_array_equal(got, want)
 
 
-@pytest.mark.parametrize("inter,M", [(8448, 3), (9728, 17), (12288, 33), (9728, 60), (8448, 64)])
+@pytest.mark.parametrize("inter,M", [(4096, 20), (6144, 5), (6400, 64), (8448, 3), (9728, 17), (12288, 33), (9728, 60),
+                                     (12544, 50)])
 def test_target_layer_wide_intermediate(cuda, inter, M):
-    """Intermediate sizes whose gate / up pair runs in blocks of six tiles (48
-    features; 9728 leaves the last block 32), at each row tile count.  With a
+    """Intermediate sizes whose gate / up pair runs in blocks of two to six half
+    tiles of 8 features, with and without a short last block (6400, 9728) and
+    beyond one block per CU (12544), at each row tile count.  With a
     zero o_proj the layer adds the MLP of x alone, so the cache's rounding stays
     out: the file's 2e-5 of an fp32 cache against 64 bits."""
     cfg = TargetConfig(hidden_size=512, num_heads=4, num_kv_heads=2, head_dim=128, intermediate_size=inter)

@@ -639,17 +639,19 @@ __device__ __forceinline__ void sk_fix_last(const SkArgs& a, int cb, float* s_c,
   sk_epi_run<TW, QKV>(a, s_c, s_inv, cb, 0, 16, ops);
 }
 
-// PE: the SiLU pair with K unsplit (ks = 1): the block owns its 32 act
-// features outright, so instead of a partial it runs the pair's epilogue
-// itself (row scale from the ss parts, SiLU(gate) * up, the next projection's
+// PE: the SiLU pair with K unsplit (ks = 1) over half tiles of 8 features:
+// rows 0..7 of an A operand are their gate rows, rows 8..15 their up rows, so
+// G of them make a block of 8 G features and the features divide over the CUs
+// in steps of 8.  The block owns its act features outright, so instead of a
+// partial it runs the pair's epilogue itself (row scale from the ss parts, SiLU(gate) * up, the next projection's
 // activations), and no fix-up launch follows.
 // FTW > 0 (MT = 1): the fix-up of column ranges of 64 FTW runs in this launch
 // (sk_fix_last), with the QKV head epilogue when FQKV.
-// G: column tiles per block (even; other than kMwG with PE only).
+// G: column tiles (PE: half tiles) per block.
 template <int MT, bool PE = false, int FTW = 0, bool FQKV = false, int G = kMwG>
 __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
   static_assert(FTW == 0 || (MT == 1 && !PE), "the fix-up in the GEMM takes one row tile");
-  static_assert(G == kMwG || (PE && G % 2 == 0), "gate / up tile pairs");
+  static_assert(G == kMwG || PE, "other block widths: the pair with K unsplit");
   constexpr int FB = 16 * G, LDR = FB + 4;
   typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(16))) float s_red[4][64 * LDR];
@@ -663,6 +665,12 @@ __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
   const uint16_t* wp[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
+    if constexpr (PE) {  // lane l: gate (l % 16 < 8) or up row 8 h + l % 8 at k group l / 16
+      const int h = min(cg * G + g, a.N / 16 - 1), lm = lane % 16;
+      wp[g] = (lm < 8 ? a.w[0] : a.w[1]) +
+              (static_cast<int64_t>(h >> 1) * S * 64 + (h & 1) * 8 + lm % 8 + 16 * (lane / 16)) * 8;
+      continue;
+    }
     const int tau = cg * G + g;
     int tb = pair ? ((tau & 1) ? a.N / 2 : 0) + 64 * (tau >> 3) + 16 * ((tau >> 1) & 3) : 16 * tau;
     tb = min(tb, ((a.N + 15) / 16 - 1) * 16);
@@ -739,8 +747,8 @@ __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
   __syncthreads();
   if constexpr (PE) {
     // four waves summed in order into wave 0's tile, then the pair epilogue
-    // of thread (row m, 8 act features from g * 8, then 32 further): gate at
-    // column 32 (f / 16) + f % 16 of the tile, up 16 columns further
+    // of thread (row m, the 8 act features of half tiles g0, g0 + 4): gate at
+    // columns 16 g .. + 7, up 8 columns further
     for (int e = t * 4; e < a.M * FB; e += 256 * 4) {
       const int r = e / FB, c = e % FB;
       float4 v = *reinterpret_cast<const float4*>(&s_red[0][r * LDR + c]);
@@ -771,8 +779,7 @@ __global__ __launch_bounds__(256) void k_mm_wave(SkArgs a) {
       float z[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int f = g * 8 + e, gc = (f / 16) * 32 + f % 16;
-        const float gv = s_red[0][m * LDR + gc] * inv, uv = s_red[0][m * LDR + gc + 16] * inv;
+        const float gv = s_red[0][m * LDR + g * 16 + e] * inv, uv = s_red[0][m * LDR + g * 16 + 8 + e] * inv;
         z[e] = gv / (1.f + expf(-gv)) * uv;
       }
       uint4 hi, lo;
@@ -926,22 +933,23 @@ static int launch_wave(SkArgs g, int fix_tw, hipStream_t s) {
   if (g.epi == kSkSiluPair && fix_tw == 2 && g.xa_next && !g.out && g.N / (16 * kMwG) >= 128 &&
       g.n_ss <= 4 * kSsMax) {
     g.ks = 1;
-    // blocks of four tiles; of six where that many would put a second block on
-    // some of the 256 CUs, which then set the launch's end, and six put one on
-    // each at most: 2 x 9728 x 2560 at 60 rows 33.1 us in 304 blocks, 22.4 in
-    // 203 (4.4 TB/s).  At 192 blocks of four (2 x 6144 features) six would
-    // leave half of the CUs idle.
+    // as many half tiles per block (two to six) as put one block on each of the
+    // 256 CUs; beyond six, six and several blocks per CU.  In blocks of 32
+    // features, 304 for 2 x 9728 x 2560 doubled up some CUs, which set the
+    // launch's end (60 rows: 33.1 us), and 192 for 2 x 6144 x 2048 left 64 idle
+    // (15.1 us); 244 and 256 blocks of 8-feature steps: 22.9 and 13.8 us (4.4 and
+    // 3.6 TB/s).
     constexpr int kCus = 256;
-    const int n4 = g.N / (16 * kMwG), n6 = (g.N + 95) / 96;
-    const bool six = n4 > kCus && n6 <= kCus;
-    const dim3 grid1(six ? n6 : n4, 1);
-#define WC_MWP(MT)                                                                                \
-  do {                                                                                            \
-    if (six)                                                                                      \
-      hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 6>), grid1, dim3(256), 0, s, g);          \
-    else                                                                                          \
-      hipLaunchKernelGGL((k_mm_wave<MT, true>), grid1, dim3(256), 0, s, g);                       \
-  } while (0)
+    const int tiles = g.N / 16, gt = std::min(6, (tiles + kCus - 1) / kCus);
+    const dim3 grid1((tiles + gt - 1) / gt, 1);
+#define WC_MWP(MT)                                                                                              \
+  switch (gt) {                                                                                                 \
+    case 2: hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 2>), grid1, dim3(256), 0, s, g); break;           \
+    case 3: hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 3>), grid1, dim3(256), 0, s, g); break;           \
+    case 4: hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 4>), grid1, dim3(256), 0, s, g); break;           \
+    case 5: hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 5>), grid1, dim3(256), 0, s, g); break;           \
+    default: hipLaunchKernelGGL((k_mm_wave<MT, true, 0, false, 6>), grid1, dim3(256), 0, s, g); break;          \
+  }
     switch ((g.M + 15) / 16) {
       case 1: WC_MWP(1); break;
       case 2: WC_MWP(2); break;
