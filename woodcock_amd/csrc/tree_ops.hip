@@ -133,18 +133,6 @@ __global__ void k_td_begin(TreeDraftState* st, const int32_t* __restrict__ root_
   }
 }
 
-// Largest key over the block (every thread receives it).
-__device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v, unsigned long long* red) {
-  v = wave_max_u64(v);
-  __syncthreads();
-  if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = v;
-  __syncthreads();
-  unsigned long long b = 0;
-#pragma unroll
-  for (int w = 0; w < kTdThreads / kWave; ++w) b = red[w] > b ? red[w] : b;
-  return b;
-}
-
 // Wave-wide maximum of u32 keys by DPP moves; every lane receives it.
 __device__ __forceinline__ uint32_t wave_max_u32_dpp(uint32_t v) {
   auto mv = [](uint32_t x, auto ctrl, auto mask) {

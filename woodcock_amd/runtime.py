@@ -14,8 +14,8 @@ from . import _lib
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 # A short call is bound by what the host does before the launch (the greedy
-# verify of 5 rows: 7 us of kernel under 16 us per call), so the plumbing of
-# every call stays off torch's Stream and device objects and ctypes' wrappers:
+# verify of 5 rows: 7 us of kernel in 16.6 us per call, 7.7 now), so the plumbing
+# of every call stays off torch's Stream and device objects and ctypes' wrappers:
 # handles are plain ints (None for the null stream).
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # absent in a torch built without a GPU
 
